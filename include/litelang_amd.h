@@ -240,7 +240,8 @@ int ll_assign_slots(int32_t* req_to_tokens, int64_t req_to_tokens_stride, const 
 
 /* ------------------------------------------------------------------- GEMM */
 
-/* Prefill tile GEMMs (256 x 256 output tiles on MFMA, see gemm_tiles.hip).
+/* Prefill tile GEMMs (256 x 256 to 128 x 128 output tiles on MFMA by shape,
+ * see gemm_tiles.hip).
  * ll_gemm_tiled: Y[M, N] = T(X[M, K] . W[N, K]^T + bias[N]) in bf16/fp16 with
  * fp32 accumulation; needs N % 4 == 0, K % 32 == 0 and 16-byte aligned rows.
  * Replaces torch.addmm / torch.mm of the reference's prefill projections
@@ -250,6 +251,11 @@ int ll_gemm_tiled_supported(int64_t M, int64_t N, int64_t K, int dtype);
 int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t ldw, const void* bias,
                   void* Y, int64_t ldy, int64_t M, int64_t N, int64_t K, int dtype,
                   hipStream_t stream);
+
+/* Workspace with which ll_gemm (M > 64) and ll_gemm_i8_tiled_ws split the K of
+ * a product with few output tiles over the CUs (elem_bytes 2: bf16/fp16, 1:
+ * int8); 0 where they do not split. With less they run one split. */
+int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K, int64_t elem_bytes);
 
 /* Copy of a [gate; up] weight ([2I, K], I % 128 == 0, elem_bytes 2 or 1)
  * with its rows interleaved in 64-row blocks (gate c..c+63, up c..c+63,
@@ -277,6 +283,12 @@ int ll_gemm_i8_tiled(const int8_t* Xq, int64_t ldx, const float* s_tok, const in
                      int64_t ldw, const void* s_ch, int s_ch_dtype, const void* bias, void* Y,
                      int64_t ldy, int64_t M, int64_t N, int64_t K, int out_dtype,
                      hipStream_t stream);
+/* ll_gemm_i8_tiled with a workspace of ll_gemm_tiles_workspace_size(M, N, K, 1)
+ * bytes (smaller or null: as ll_gemm_i8_tiled); the same bits either way. */
+int ll_gemm_i8_tiled_ws(const int8_t* Xq, int64_t ldx, const float* s_tok, const int8_t* Wq,
+                        int64_t ldw, const void* s_ch, int s_ch_dtype, const void* bias, void* Y,
+                        int64_t ldy, int64_t M, int64_t N, int64_t K, int out_dtype,
+                        void* workspace, int64_t workspace_bytes, hipStream_t stream);
 /* The raw int32 sums of the same product (Y int32 [M, N]). */
 int ll_gemm_i8_i32_tiled(const int8_t* Xq, int64_t ldx, const int8_t* Wq, int64_t ldw,
                          int32_t* Y, int64_t ldy, int64_t M, int64_t N, int64_t K,
@@ -302,7 +314,8 @@ int ll_gemm_i8_gate_up_silu_tiled(const int8_t* Xq, int64_t ldx, const float* s_
  * [in, out]; this library keeps [out, in] so both MFMA operands stream
  * 16-byte k-contiguous rows). X rows may be strided; Y is written with
  * row stride ldy. For M <= 64 with narrow N the product is split over K and
- * needs a workspace of ll_gemm_workspace_size(M, N, K) bytes (0 otherwise). */
+ * needs a workspace of ll_gemm_workspace_size(M, N, K) bytes (0 otherwise).
+ * For M > 64 a workspace is optional (ll_gemm_tiles_workspace_size). */
 int64_t ll_gemm_workspace_size(int64_t M, int64_t N, int64_t K);
 int ll_gemm(const void* X, int64_t ldx, const void* W, int64_t ldw, const void* bias, void* Y,
             int64_t ldy, int64_t M, int64_t N, int64_t K, int dtype, void* workspace,

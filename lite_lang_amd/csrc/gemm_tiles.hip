@@ -5,32 +5,37 @@
 // (the reference's SmoothQuant module has no forward, quantize/smooth_quant/
 // layer.py:19-59).
 //
-// One workgroup (8 waves, two per SIMD) per CU computes 256 x 256 output
-// tiles one after the other (a persistent grid):
-//   * stages of 64 bytes of K per row (32 bf16/fp16 or 64 int8) for the
-//     tile's 256 weight rows and 256 activation rows (32 KB) are copied
-//     global -> LDS with global_load_lds_dwordx4 (no VGPR staging) into a
-//     ring of five stage buffers (160 KB), four stages in flight ahead of
-//     the one being multiplied; the ring runs on from one tile into the
-//     next, so no tile after the first waits for its first stages;
-//   * a finished tile's outputs are stored with buffer stores that nothing
-//     waits for until the ring's own waits reach them, a few stages into
-//     the next tile;
+// One workgroup (8 waves, two per SIMD) per CU works off (k split, output
+// tile) items one after the other (a persistent grid); tiles are 256 x 256,
+// 256 x 128 or 128 x 128 by shape (plan_tiles):
+//   * stages of 128 bytes of K per row (64 bf16/fp16 or 128 int8) of the
+//     tile's weight and activation rows are copied global -> LDS with
+//     global_load_lds_dwordx4 (no VGPR staging) into a ring of two to four
+//     stage buffers that runs on from one item into the next. A row's 128
+//     bytes are one cache line: 64-byte rows fetched every line twice and
+//     fed a CU at 56 GB/s with all CUs reading, 128-byte rows at 134 GB/s;
+//   * the ring is refilled in pieces of 128 rows, each as soon as both wave
+//     groups have read it, so the copies lead the reads by more than a stage
+//     although the 256 x 256 form holds only two stages;
+//   * a finished item's rows are turned through the wave's own LDS and stored
+//     as whole 128-byte segments with buffer stores that nothing waits for
+//     until the ring's own waits reach them;
 //   * the 16-byte chunks of every LDS row are XOR-swizzled (tile_swz) so
-//     the MFMA operand reads (16 rows x 16 B per 16 lanes) hit distinct
-//     banks;
-//   * each wave multiplies 128 weight rows by 64 activation rows with
-//     v_mfma_f32_32x32x16_bf16 (v_mfma_i32_32x32x32_i8 for int8) as
+//     the MFMA operand reads hit distinct banks;
+//   * each wave multiplies 64 or 128 weight rows by 32 or 64 activation rows
+//     with v_mfma_f32_16x16x32 (v_mfma_i32_16x16x64_i8 for int8) as
 //     C^T = W . X^T: the weight rows are the MFMA's row operand, so every
-//     lane ends with runs of 4 consecutive output columns of one token row
-//     (8-byte stores) in 8 accumulator blocks of 32 x 32. The second wave
-//     on each SIMD issues while the first waits on LDS or the barrier (one
-//     wave per SIMD reaches about 150 B/clk of LDS reads per CU, two about
-//     240);
+//     lane ends with runs of 4 consecutive output columns of one token row.
+//     At large sizes the card is power-bound (1.6 GHz, the matrix pipes busy
+//     85% of the cycles), and the 16 x 16 form, which moves half the
+//     accumulator registers per product, runs 6% faster than 32 x 32;
 //   * the grid is XCD-aware: the workgroups the dispatcher deals to one XCD
-//     take a contiguous range of tiles in groups of 1, 2 or 4 row tiles by
-//     shape (tile_group_m), round robin, so tiles sharing activation or
-//     weight rows run together on one L2.
+//     take a contiguous range of items, tiles in groups of 1, 2 or 4 row
+//     tiles by shape (tile_group_m), round robin, so tiles sharing activation
+//     or weight rows run together on one L2.
+// Measured (bf16, one launch): gate/up + SiLU at M = 24,000 (3B) 1790 -> 1736
+// us (1247 TFLOP/s), down_proj 930 -> 780 (1388), qkv 272 -> 202; down_proj
+// at M = 333 204 -> 33 us.
 // Epilogues: the model dtype with an optional bias; SiLU_and_Mul of a
 // gate/up weight interleaved in 64-row blocks (ll_gemm_interleave_gate_up),
 // with the rounding sequence of ll_silu_and_mul; int8 sums dequantised as
@@ -38,43 +43,74 @@
 // raw int32 sums.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "ll_common.h"
 
 namespace {
 
-constexpr int kT = 256;        // output tile: 256 activation rows x 256 weight rows
-constexpr int kRB = 64;        // bytes of K per row per stage
-constexpr int kStageB = 2 * kT * kRB;  // 32 KB: weight rows, then activation rows
-constexpr int kNst = 5;        // stage buffers (160 KB of LDS)
+constexpr int kRB = 128;       // bytes of K per row per stage: one cache line
+constexpr int kKUnit = 64;     // K spans a multiple of this many bytes
+constexpr int kPlanCus = 256;   // CUs the workspace query plans for
+constexpr int kMinSplitStages = 6;  // stages a k split holds at least
+constexpr int kPieceB = 128 * kRB;  // a piece: 128 rows of one operand (16 KB)
 constexpr int kWaves = 8;      // two per SIMD
 constexpr int kThreads = 64 * kWaves;
-constexpr int kPW = 4;         // 32-row weight blocks per wave (128 rows: wave column wn of 2)
-constexpr int kQX = 2;         // 32-row activation blocks per wave (64 rows: wave row wm of 4)
-constexpr int kNMf = kPW * kQX;  // MFMAs per wave per k-step
-constexpr int kDmaW = 2 * kT * kRB / 16 / kThreads;  // 16-byte copies per lane per stage
-static_assert(2 * 32 * kPW == kT && 4 * 32 * kQX == kT && kWaves == 8, "wave grid 2 x 4");
-static_assert(kDmaW == 4, "copy geometry: 4 instructions of 16 rows per wave per stage");
+constexpr int kDma = 2;        // 16-byte copies per lane per piece
 
-enum { EPI_STORE = 0, EPI_SILU = 1, EPI_DEQ = 2, EPI_DEQ_SILU = 3, EPI_I32 = 4 };
+// Tile geometry: NWP pieces of 128 weight rows by NXP pieces of 128
+// activation rows (W0, W1 and X0, X1 below). The phases of stage t, in order,
+// each reading pieces from LDS and then multiplying:
+//   2 x 2 (256 x 256): W0(t) X1(t) -> W0 X0, W0 X1; W1(t) X0(t + 1) -> W1 X0, W1 X1
+//   2 x 1 (256 x 128): W0(t) X0(t) -> W0 X0; W1(t) -> W1 X0
+//   1 x 1 (128 x 128): W0(t) X0(t) -> W0 X0
+// The 2 x 2 form reads X0 a stage ahead (two register sets, by stage parity),
+// so that both phases read 12 fragments per lane for 16 MFMAs: the time of
+// the reads and of the other group's MFMAs is the same. A piece's slot in
+// the stage buffer is its place in that order.
+template <int NWP_, int NXP_> struct TileGeo {
+  static constexpr int NWP = NWP_, NXP = NXP_;
+  static constexpr int TN = 128 * NWP, TM = 128 * NXP;
+  static constexpr int kPieces = NWP + NXP;
+  static constexpr bool kAhead = kPieces == 4;  // X0 is read a stage ahead
+  static constexpr int kPh = NWP;               // phases per stage
+  static constexpr int kStageB = kPieces * kPieceB;
+  static constexpr int kNst = kPieces == 4 ? 2 : kPieces == 3 ? 3 : 4;  // stage buffers
+  static constexpr int kEpB = (160 * 1024 - kNst * kStageB) / kWaves;   // epilogue bytes per wave
+  static constexpr size_t kLds = (size_t)kNst * kStageB + (size_t)kWaves * kEpB;
+  static constexpr bool is_w(int q) { return q == 0 || q == 2; }
+  static constexpr int w_half(int q) { return q / 2; }
+  static constexpr int x_half(int q) { return kAhead && q == 1 ? 1 : 0; }
+  // pieces of phase ph: first(ph) .. last(ph)
+  static constexpr int first(int ph) { return 2 * ph; }
+  static constexpr int last(int ph) { return 2 * ph + 1 < kPieces ? 2 * ph + 1 : kPieces - 1; }
+  static constexpr int copies(int ph) { return (last(ph) - first(ph) + 1) * kDma; }
+  // copies a wave has issued after those of phase q's pieces when the pieces
+  // are about to be read (the counted wait before the read)
+  static constexpr int wait_cnt(int q) {
+    int n = 0;
+    for (int i = 1; i <= kNst * kPh - 2; ++i) n += copies((q + i) % kPh);
+    return n;
+  }
+};
 
-typedef float f32x16v __attribute__((ext_vector_type(16)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
+enum { EPI_STORE = 0, EPI_SILU = 1, EPI_DEQ = 2, EPI_DEQ_SILU = 3, EPI_I32 = 4, EPI_PART = 5 };
+
 template <typename T> struct TileOp;
-template <> struct TileOp<__bf16> { typedef bf16x8 V; typedef f32x16v Acc; };
-template <> struct TileOp<_Float16> { typedef f16x8 V; typedef f32x16v Acc; };
-template <> struct TileOp<int8_t> { typedef i32x4 V; typedef i32x16 Acc; };
+template <> struct TileOp<__bf16> { typedef bf16x8 V; typedef f32x4 Acc; };
+template <> struct TileOp<_Float16> { typedef f16x8 V; typedef f32x4 Acc; };
+template <> struct TileOp<int8_t> { typedef i32x4 V; typedef i32x4 Acc; };
 
-// 32 x 32 output block, 16 bf16/fp16 (32 int8) of K per instruction: lane l
-// supplies row (or column) l % 32 and the 16-byte K chunk l / 32
-__device__ __forceinline__ f32x16v tile_mma(bf16x8 a, bf16x8 b, f32x16v c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+// 16 x 16 output block, 32 bf16/fp16 (64 int8) of K per instruction: lane l
+// supplies row (or column) l % 16 and the 16-byte K chunk l / 16.
+__device__ __forceinline__ f32x4 tile_mma(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f32x16v tile_mma(f16x8 a, f16x8 b, f32x16v c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+__device__ __forceinline__ f32x4 tile_mma(f16x8 a, f16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ i32x16 tile_mma(i32x4 a, i32x4 b, i32x16 c) {
-  return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+__device__ __forceinline__ i32x4 tile_mma(i32x4 a, i32x4 b, i32x4 c) {
+  return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
 // 16 B global -> LDS copy of one lane (lane i lands at lds + 16 i); kept out of
@@ -98,410 +134,569 @@ __device__ __forceinline__ void tile_barrier() {
 struct TileArgs {
   const char* X; int64_t ldx_b;   // activation rows (K contiguous), row stride in bytes
   const char* W; int64_t ldw_b;   // weight rows [N][K] (EPI_SILU*: interleaved gate/up)
-  int M, N, K_b;                  // K in bytes
-  int tiles_m, tiles_n;
+  int M, N;
+  int nk;                         // stages of the whole K
+  int kps;                        // stages per k split (the last split may have fewer)
+  int half;                       // the last stage of K holds 64 bytes per row, not 128
+  int tiles_m, tiles_n, splits;
   int group_m;                    // row tiles per group of the tile order (tile_group_m)
   void* Y; int64_t ldy;           // output, row stride in elements of the output type
   int y_bytes;                    // bytes from Y to the end of its last row (< 2^31)
+  int64_t split_b;                // bytes between the outputs of consecutive k splits
+  int wide;                       // output rows and column counts allow 16-byte stores
   const void* bias;               // [N] in the model dtype, or null
   const float* s_tok;             // int8: activation scale per row [M]
   const void* s_ch; int s_ch_dtype;  // int8: weight scale per channel [N]
 };
 
-// Swizzle of the 16-byte chunks of 64-byte LDS row r (an involution on
-// 0..3): chunk c of row r sits at chunk c ^ ((r / 4) % 4). Measured with
-// ds_read_b128 over the fragment pattern (32 rows x one chunk per 32
-// lanes): about 205 B/clk per CU, as for contiguous reads, against 116 B/clk
-// for a swizzle on (r / 2) ^ (r / 8) and 63 B/clk unswizzled.
-__device__ __forceinline__ int tile_swz(int r) { return (r >> 2) & 3; }
-// LDS byte offset of chunk c (16 B) of tile row r within a stage half
-__device__ __forceinline__ int tile_lds_off(int r, int c) { return r * kRB + ((c ^ tile_swz(r)) << 4); }
+// Swizzle of the 16-byte chunks of 128-byte LDS row r (an involution on
+// 0..7): chunk c of row r sits at chunk c ^ ((r / 2) % 8), so 16 consecutive
+// rows read at one chunk index cover all 64 banks once.
+__device__ __forceinline__ int tile_swz(int r) { return (r >> 1) & 7; }
 
 // Output tile (m0, n0) of tile t of the grouped order: groups of group_m row
 // tiles, each group's column tiles in order with its row tiles innermost.
+template <typename G>
 __device__ __forceinline__ void tile_coords(const TileArgs& a, int t, int& m0, int& n0) {
   const int gsz = a.group_m * a.tiles_n;
   const int grp = t / gsz, rin = t - grp * gsz;
   const int gm = min(a.group_m, a.tiles_m - grp * a.group_m);
-  m0 = (grp * a.group_m + rin % gm) * kT;
-  n0 = (rin / gm) * kT;
+  m0 = (grp * a.group_m + rin % gm) * G::TM;
+  n0 = (rin / gm) * G::TN;
 }
 
-// Row tiles per group of the tile order, by shape class, as measured on the
-// 3B prefill projections at M = 24,000 (group sizes 1, 2, 4 and 8, libraries
-// interleaved, best of 4 rounds): wide outputs (gate/up, 86 column tiles)
-// 4 (1788 us against 1813 with 2 and 1886-1898 with 1 or 8); long K
-// (down_proj, 172 stages) 1 (916 against 953 with 2); the narrow short-K
-// shapes (qkv, o_proj) level at every size (2).
-int tile_group_m(int64_t tiles_n, int64_t nk) {
-  if (tiles_n >= 32) return 4;
-  if (nk >= 128) return 1;
-  return 2;
-}
-
-// Buffer store of 4 consecutive outputs. A lane whose offset is kTileNoStore
-// (beyond the buffer's size) stores nothing, so every wave issues the same
-// number of store instructions for every tile, edges included: the copy
-// ring's vmcnt waits count them. The empty asm keeps the compiler from
-// merging stores, which would change that count.
+// A store lane whose offset is kTileNoStore (beyond the buffer's size) stores
+// nothing, so every wave issues the same number of store instructions for
+// every tile, edges included: the copy ring's vmcnt waits count them. The
+// empty asm keeps the compiler from merging stores, which would change that
+// count.
 constexpr uint32_t kTileNoStore = 0x80000000u;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-template <typename TO>
-__device__ __forceinline__ void tile_store4(__amdgpu_buffer_rsrc_t r, uint32_t off, const TO (&o)[4]) {
-  typedef TO V4 __attribute__((ext_vector_type(4)));
-  const V4 v = {o[0], o[1], o[2], o[3]};
-  if constexpr (sizeof(TO) == 2) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, 0);
-  } else {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, 0);
-  }
-  asm volatile("" ::: "memory");
-}
 
-// Raw bits of the scales of `n` consecutive channels from i (fp32 bits, or a
-// zero-extended fp16 / bf16 code; ll_scale_bits_to_f32 converts them). The
-// dtype branch is taken once for all the loads, so none waits for another.
+// Scales of channels i[j] .. i[j] + 3 as fp32. The dtype branch is taken once
+// for all the loads and conversions, so one wait serves them all.
 template <int n>
-__device__ __forceinline__ void tile_scale_bits(const void* s, int dtype, const int (&i)[n],
-                                                uint32_t (&b)[n][4]) {
+__device__ __forceinline__ void tile_scales(const void* s, int dtype, const int (&i)[n],
+                                            float (&f)[n][4]) {
   if (dtype == LL_F32) {
 #pragma unroll
     for (int j = 0; j < n; ++j)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) b[j][k] = ((const uint32_t*)s)[i[j] + k];
+      for (int k = 0; k < 4; ++k) f[j][k] = *(const float*)((const char*)s + (uint32_t)(4 * (i[j] + k)));
   } else {
+    uint32_t b[n][4];
 #pragma unroll
     for (int j = 0; j < n; ++j)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) b[j][k] = ((const uint16_t*)s)[i[j] + k];
+      for (int k = 0; k < 4; ++k) b[j][k] = *(const uint16_t*)((const char*)s + (uint32_t)(2 * (i[j] + k)));
+    if (dtype == LL_F16) {
+#pragma unroll
+      for (int j = 0; j < n; ++j)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f[j][k] = ll_scale_bits_to_f32(b[j][k], LL_F16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < n; ++j)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f[j][k] = ll_scale_bits_to_f32(b[j][k], LL_BF16);
+    }
   }
 }
 
-template <typename T, typename TO, int EPI>
+// Every lambda of the kernel is inlined before the arrays it captures are
+// split into registers (left to the inliner, they stay in scratch memory).
+#define LL_INLINE __attribute__((always_inline))
+
+template <typename T, typename TO, int EPI, typename G>
 __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
   typedef typename TileOp<T>::V V;
   typedef typename TileOp<T>::Acc Acc;
   constexpr bool kSilu = EPI == EPI_SILU || EPI == EPI_DEQ_SILU;
-  constexpr int kStores = kSilu ? 16 : 32;  // store instructions per wave per tile
+  constexpr int kPh = G::kPh, kNst = G::kNst, NWP = G::NWP, NXP = G::NXP;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  // ---- tiles of this workgroup. XCD x (= blockIdx % 8, up to a launch-wide
-  // rotation) owns tiles x * per .. x * per + per - 1 of the grouped order;
-  // its gridDim / 8 workgroups (one per CU) take them round robin, so the
-  // tiles in flight on one XCD at any time are consecutive in that order.
+  // ---- work items of this workgroup: (k split, output tile), splits
+  // outermost. XCD x (= blockIdx % 8, up to a launch-wide rotation) owns
+  // items x * per .. x * per + per - 1; its gridDim / 8 workgroups (one per
+  // CU) take them round robin, so the tiles in flight on one XCD at any time
+  // are consecutive in the grouped order and share rows in its L2.
   const int tiles = a.tiles_m * a.tiles_n;
-  const int per = (tiles + 7) / 8;
+  const int items = tiles * a.splits;
+  const int per = (items + 7) / 8;
   const int g8 = (int)(gridDim.x >> 3);
-  const int t_first = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  const int t_end = min((int)(blockIdx.x & 7) * per + per, tiles);
-  if (t_first >= t_end) return;
-  const int ntl = (t_end - t_first + g8 - 1) / g8;  // tiles of this workgroup
-  const int nk = a.K_b / kRB;                        // stages per tile
-  const int total = ntl * nk;                        // stages this workgroup multiplies
+  const int i_first = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  const int i_end = min((int)(blockIdx.x & 7) * per + per, items);
+  if (i_first >= i_end) return;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wn = wave & 1, wm = wave >> 1;
 
-  // ---- copy stream: the stages of all of this workgroup's tiles in order,
-  // so a tile's first stages are copied while the previous tile is still
-  // being multiplied. Instruction u of this wave is copy j = u * 8 + wave of
-  // the stage's 32; copy j covers LDS rows 16 * (j % 16) .. + 15 of the
-  // weight half (j < 16) or the activation half; lane -> row + l/4, LDS
-  // chunk l % 4.
-  const int crow = lane >> 2;
-  uint32_t soff[kDmaW];  // byte offsets of this lane's copy sources (rows clamped into range)
-  auto set_sources = [&](int t) {
+  // ---- copy stream: the pieces of all of this workgroup's stages in phase
+  // order, running on from one item into the next. Instruction u of this wave
+  // copies rows 8 j .. 8 j + 7 (j = 8 u + wave) of a piece; lane -> row
+  // 8 j + l / 8, LDS chunk l % 8, that is global chunk (l % 8) ^ swizzle,
+  // the same for every piece. Row i of W piece h is tile row
+  //   2 x *: (2 (i / 64) + h) * 64 + i % 64 (64-row block 2 wn + h for wave column wn);
+  //   1 x *: i, or for the SiLU forms ((i / 32) % 2) * 64 + (i / 64) * 32 + i % 32,
+  // so that a wave holds a gate channel and its up channel.
+  const int gch = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
+  const uint32_t tail_adj = gch >= 4 ? 64u : 0u;  // half stage: chunks past K re-read the row's last 64 B
+  uint32_t soff[G::kPieces][kDma];
+  // 32-bit product and sum (the spans are below 4 GiB), kept apart: their
+  // 64-bit multiply-add would hold a register pair per offset
+  auto row_off = [&](int row, uint32_t ld) LL_INLINE {
+    uint32_t o = (uint32_t)row * ld;
+    asm volatile("" : "+v"(o));
+    return o + (uint32_t)gch * 16;
+  };
+  auto set_sources = [&](int t) LL_INLINE {
     int m0, n0;
-    tile_coords(a, t, m0, n0);
+    tile_coords<G>(a, t, m0, n0);
+    int sl = lane;  // as a value of its own (no row number is held through the main loop)
+    asm volatile("" : "+v"(sl));
 #pragma unroll
-    for (int u = 0; u < kDmaW; ++u) {
-      const int j = u * kWaves + wave;
-      const int r = 16 * (j & 15) + crow;
-      const int gch = (lane & 3) ^ tile_swz(r);
-      if (j < 16) soff[u] = (uint32_t)((int64_t)min(n0 + r, a.N - 1) * a.ldw_b + gch * 16);
-      else soff[u] = (uint32_t)((int64_t)min(m0 + r, a.M - 1) * a.ldx_b + gch * 16);
+    for (int q = 0; q < G::kPieces; ++q)
+#pragma unroll
+      for (int u = 0; u < kDma; ++u) {
+        const int i = 8 * (8 * u + wave) + (sl >> 3);
+        if (G::is_w(q)) {
+          int r;
+          if constexpr (NWP == 2) r = (2 * (i >> 6) + G::w_half(q)) * 64 + (i & 63);
+          else if constexpr (kSilu) r = ((i >> 5) & 1) * 64 + (i >> 6) * 32 + (i & 31);
+          else r = i;
+          soff[q][u] = row_off(min(n0 + r, a.N - 1), (uint32_t)a.ldw_b);
+        } else {
+          const int r = G::x_half(q) * 128 + i;
+          soff[q][u] = row_off(min(m0 + r, a.M - 1), (uint32_t)a.ldx_b);
+        }
+      }
+  };
+  // cursor of the copies: item, its first stage, stage within it, ring buffer
+  int iss_i = i_first, iss_k = 0, iss_ke = 0, iss_buf = 0;
+  auto iss_item = [&]() LL_INLINE {
+    const int sp = iss_i / tiles;
+    set_sources(iss_i - sp * tiles);
+    iss_k = sp * a.kps;
+    iss_ke = min(iss_k + a.kps, a.nk);
+  };
+  iss_item();
+  // Copies of read phase rp of the cursor's stage; the last phase moves the
+  // cursor on (before X0 where that is read a stage ahead). Past the last
+  // item every lane copies the operand's first bytes (in bounds, never read,
+  // one line), so each wave issues the same number of copies in every phase.
+  auto issue_piece = [&](auto qc) LL_INLINE {
+    constexpr int q = decltype(qc)::value;
+    const bool past = iss_i >= i_end;
+    const uint32_t pmask = past ? 0u : ~0u;
+    const uint32_t tadj = (a.half && iss_k == a.nk - 1) ? tail_adj : 0u;
+    const int64_t kb = past ? 0 : (int64_t)iss_k * kRB;
+#pragma unroll
+    for (int u = 0; u < kDma; ++u) {
+      uint32_t o = (soff[q][u] - tadj) & pmask;
+      asm volatile("" : "+v"(o));  // no 64-bit form of it is held through the loop
+      tile_dma16((G::is_w(q) ? a.W : a.X) + kb + o,
+                 smem + iss_buf * G::kStageB + q * kPieceB + (8 * u + wave) * 1024);
     }
   };
-  set_sources(t_first);
-  int iss_j = 0, iss_ks = 0, iss_buf = 0;  // tile (local index), stage and ring buffer of the next copies
-  // Copies past the last tile repeat its last stage (in bounds, never read),
-  // so every wave's vmcnt arithmetic is the same in every iteration.
-  auto issue = [&]() {
-    const int ks = iss_j < ntl ? iss_ks : nk - 1;
-#pragma unroll
-    for (int u = 0; u < kDmaW; ++u) {
-      const int j = u * kWaves + wave;
-      char* dst = smem + iss_buf * kStageB + (j >> 4) * (kT * kRB) + (j & 15) * 1024;
-      tile_dma16((j < 16 ? a.W : a.X) + (int64_t)ks * kRB + soff[u], dst);
-    }
+  auto issue_next = [&]() LL_INLINE {
     iss_buf = iss_buf == kNst - 1 ? 0 : iss_buf + 1;
-    if (iss_j < ntl && ++iss_ks == nk) {
-      iss_ks = 0;
-      if (++iss_j < ntl) set_sources(t_first + iss_j * g8);
+    if (iss_i < i_end && ++iss_k == iss_ke) {
+      iss_i += g8;
+      if (iss_i < i_end) iss_item();
     }
+  };
+  auto issue = [&](auto rpc) LL_INLINE {
+    constexpr int rp = decltype(rpc)::value;
+    issue_piece(std::integral_constant<int, G::first(rp)>{});
+    if constexpr (rp == kPh - 1 && G::kAhead) issue_next();
+    if constexpr (G::last(rp) > G::first(rp)) issue_piece(std::integral_constant<int, G::last(rp)>{});
+    if constexpr (rp == kPh - 1 && !G::kAhead) issue_next();
   };
 
-  Acc acc[kPW][kQX];
-  auto zero_acc = [&]() {
+  Acc acc[NWP][NXP][4][2];
+  auto zero_acc = [&]() LL_INLINE {
 #pragma unroll
-    for (int p = 0; p < kPW; ++p)
+    for (int h = 0; h < NWP; ++h)
 #pragma unroll
-      for (int q = 0; q < kQX; ++q)
+      for (int j = 0; j < NXP; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[p][q][e] = 0;
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) acc[h][j][p][q] = Acc{0, 0, 0, 0};
   };
   zero_acc();
 
-  const int lr = lane & 31, lc = lane >> 5;
-  const int wrow = wn * 128 + lr, xrow = wm * 64 + lr;
-  const int c0 = lc, c1 = 2 + lc;  // LDS chunks of k-step 0 and 1 for this lane
-  V fw[2][kPW], fx[2][kQX];
-  auto frag_w = [&](int buf, int c, int p) {
-    return *(const V*)(smem + buf * kStageB + tile_lds_off(wrow + 32 * p, c));
+  // ---- fragments: of a W piece this wave's 64 rows (wn) as four 16-row
+  // blocks, of an X piece its 32 rows (wm) as two; k step ks is LDS chunks
+  // 4 ks .. 4 ks + 3 (lane l / 16). Byte offset of k step ks in a row block
+  // of a piece: one register per k step, everything else of the address is
+  // scalar or immediate (opaque, so that no other form of it takes registers
+  // through the loop).
+  int foff[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    foff[ks] = (lane & 15) * kRB + (((4 * ks + (lane >> 4)) ^ tile_swz(lane & 15)) << 4);
+    asm volatile("" : "+v"(foff[ks]));
+  }
+  // fx[0]: X0, fx[1]: X1, fx[2]: the next stage's X0 where it is read ahead
+  V fw[2][4], fx[3][2][2];
+  auto read_w = [&](auto qc, int buf) LL_INLINE {
+    const int sb = buf * G::kStageB + decltype(qc)::value * kPieceB + wn * 64 * kRB;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) fw[ks][p] = *(const V*)(smem + (sb + foff[ks]) + 16 * p * kRB);
   };
-  auto frag_x = [&](int buf, int c, int q) {
-    return *(const V*)(smem + buf * kStageB + kT * kRB + tile_lds_off(xrow + 32 * q, c));
+  auto read_x = [&](auto qc, int buf, V (&f)[2][2]) LL_INLINE {
+    const int sb = buf * G::kStageB + decltype(qc)::value * kPieceB + wm * 32 * kRB;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) f[ks][q] = *(const V*)(smem + (sb + foff[ks]) + 16 * q * kRB);
   };
-  auto read_stage = [&](int g) {
-    const int buf = g % kNst;
+  // the pieces of phase ph of the stage in buffer buf
+  auto read_phase = [&](auto phc, int buf) LL_INLINE {
+    constexpr int ph = decltype(phc)::value;
+    if constexpr (G::kAhead && ph == 0) {
 #pragma unroll
-    for (int p = 0; p < kPW; ++p) fw[0][p] = frag_w(buf, c0, p);
-#pragma unroll
-    for (int q = 0; q < kQX; ++q) fx[0][q] = frag_x(buf, c0, q);
-#pragma unroll
-    for (int p = 0; p < kPW; ++p) fw[1][p] = frag_w(buf, c1, p);
-#pragma unroll
-    for (int q = 0; q < kQX; ++q) fx[1][q] = frag_x(buf, c1, q);
+      for (int i = 0; i < 4; ++i) fx[0][i / 2][i % 2] = fx[2][i / 2][i % 2];
+    }
+    read_w(std::integral_constant<int, G::first(ph)>{}, buf);
+    if constexpr (G::kAhead) {
+      if constexpr (ph == 0) read_x(std::integral_constant<int, 1>{}, buf, fx[1]);
+      else read_x(std::integral_constant<int, 3>{}, 1 - buf, fx[2]);
+    } else if constexpr (ph == 0) {
+      read_x(std::integral_constant<int, 1>{}, buf, fx[0]);
+    }
   };
-  auto compute = [&]() {
+  // products of phase ph; full: both k steps (a half stage has one)
+  auto multiply = [&](auto phc, bool full) LL_INLINE {
+    constexpr int h = decltype(phc)::value;
+    auto step = [&](int ks) LL_INLINE {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+      for (int j = 0; j < NXP; ++j)
 #pragma unroll
-      for (int i = 0; i < kNMf; ++i)
-        acc[i / kQX][i % kQX] = tile_mma(fw[kk][i / kQX], fx[kk][i % kQX], acc[i / kQX][i % kQX]);
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            acc[h][j][p][q] = tile_mma(fw[ks][p], fx[j][ks][q], acc[h][j][p][q]);
+    };
+    step(0);
+    if (full) step(1);
   };
 
-  // ---- epilogue of tile ep_j: acc[p][q][4g + i] = C[m][n] with
-  //   m = m0 + wm*64 + 32q + l % 32,  n = n0 + wn*128 + 32p + 8g + 4(l / 32) + i
-  const __amdgpu_buffer_rsrc_t yres =
-      __builtin_amdgcn_make_buffer_rsrc(a.Y, (short)0, a.y_bytes, 0x00020000);
-  int ep_j = 0;
-  auto epilogue = [&]() {
-    int m0, n0;
-    tile_coords(a, t_first + ep_j * g8, m0, n0);
-    ++ep_j;
-    const int mrow = m0 + wm * 64 + lr;
-    // The per-row and per-column factors are all loaded before the first
-    // store, so the wave waits for them (and for the copies in flight ahead
-    // of them) once, not once per store.
-    float st[kQX];
+  // ---- epilogue. acc[h][j][p][q][i] = C[m][n] with m = m0 + 128 j + 32 wm
+  // + 16 q + l % 16 and n = n0 + (the 64 columns of h and wn) + 16 p +
+  // 4 (l / 16) + i. A lane's run of 4 columns is 8 or 16 bytes, so the rows
+  // are turned through the wave's own piece of LDS: stores of whole 128-byte
+  // (64-byte where the piece is smaller) row segments, 16 bytes per lane.
+  constexpr int kCB = G::kEpB >= 4096 && !(kSilu && NWP == 1) ? 128 : 64;  // bytes per row segment
+  constexpr int kRowsPI = 1024 / kCB;                 // rows per store instruction
+  constexpr int kSegCols = kCB / (int)sizeof(TO);     // columns per segment
+  constexpr int kOutB = NWP * NXP * 64 * 32 * (int)sizeof(TO) / (kSilu ? 2 : 1);  // bytes per wave
+  constexpr int kStores = kOutB / 1024;
+  char* const ep = smem + kNst * G::kStageB + wave * G::kEpB;
+  auto ep_swz = [](int row) LL_INLINE { return kCB == 128 ? (row & 7) : ((row >> 1) & 3); };
+  // 4 outputs of row `row` at column c (multiple of 4) of the segment
+  auto ep_put = [&](int row, int c, const TO (&o)[4]) LL_INLINE {
+    typedef TO V4 __attribute__((ext_vector_type(4)));
+    const V4 v = {o[0], o[1], o[2], o[3]};
+    const int b = c * (int)sizeof(TO);
+    *(V4*)(ep + row * kCB + ((((b >> 4) ^ ep_swz(row)) << 4) | (b & 15))) = v;
+  };
+  // store the segment: rows mb .. mb + 31, columns nb .. nb + kSegCols - 1 of
+  // the nmax columns of the output
+  auto ep_store = [&](int el, const __amdgpu_buffer_rsrc_t& r, int mb, int nb, int nmax) LL_INLINE {
+    u32x4 v[32 / kRowsPI];
 #pragma unroll
-    for (int q = 0; q < kQX; ++q) {
-      st[q] = 1.f;
-      if constexpr (EPI == EPI_DEQ || EPI == EPI_DEQ_SILU) st[q] = a.s_tok[min(mrow + 32 * q, a.M - 1)];
+    for (int it = 0; it < 32 / kRowsPI; ++it) {
+      const int row = it * kRowsPI + el / (kCB / 16), ch = el % (kCB / 16);
+      v[it] = *(const u32x4*)(ep + row * kCB + ((ch ^ ep_swz(row)) << 4));
     }
+#pragma unroll
+    for (int it = 0; it < 32 / kRowsPI; ++it) {
+      const int m = mb + it * kRowsPI + el / (kCB / 16);
+      const int n = nb + el % (kCB / 16) * (16 / (int)sizeof(TO));
+      const uint32_t off = (uint32_t)(((int64_t)m * a.ldy + n) * (int64_t)sizeof(TO));
+      if (a.wide) {
+        __builtin_amdgcn_raw_buffer_store_b128(v[it], r, (m < a.M && n < nmax) ? off : kTileNoStore, 0, 0);
+      } else {  // 8-byte halves: rows 8-byte aligned, or a last chunk of 4 columns
+        const u32x2 lo = {v[it][0], v[it][1]}, hi = {v[it][2], v[it][3]};
+        const int n2 = n + 8 / (int)sizeof(TO);
+        __builtin_amdgcn_raw_buffer_store_b64(lo, r, (m < a.M && n < nmax) ? off : kTileNoStore, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(hi, r, (m < a.M && n2 < nmax) ? off + 8 : kTileNoStore, 0, 0);
+      }
+      asm volatile("" ::: "memory");
+    }
+  };
+  auto epilogue = [&](int item) LL_INLINE {
+    const int sp = item / tiles;
+    int m0, n0;
+    tile_coords<G>(a, item - sp * tiles, m0, n0);
+    const __amdgpu_buffer_rsrc_t yres = __builtin_amdgcn_make_buffer_rsrc(
+        (char*)a.Y + (int64_t)sp * a.split_b, (short)0, a.y_bytes, 0x00020000);
+    const int mw = m0 + wm * 32;
+    // the lane as a value of its own: nothing that follows from it is
+    // computed ahead of the main loop and held in registers through it
+    int el = lane;
+    asm volatile("" : "+v"(el));
+    const int lr = el & 15, lc = el >> 4;
+    // The per-row and per-column factors are loaded before the first store
+    // that needs them, so the wave waits for them (and for the copies in
+    // flight ahead of them) once, not once per store.
+    float st[NXP][2];
+#pragma unroll
+    for (int j = 0; j < NXP; ++j)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        st[j][q] = 1.f;
+        if constexpr (EPI == EPI_DEQ || EPI == EPI_DEQ_SILU)
+          st[j][q] = a.s_tok[min(mw + 128 * j + 16 * q + lr, a.M - 1)];
+      }
     if constexpr (!kSilu) {
       typedef TO V4 __attribute__((ext_vector_type(4)));
-      const bool has_bias = EPI != EPI_I32 && a.bias != nullptr;
-      const int ncol = n0 + wn * 128 + 4 * lc;
-      // weight blocks p per pass: the dequantising epilogue's scales take 4
-      // registers per column group, so it makes two passes
-      constexpr int kPass = EPI == EPI_DEQ ? 2 : kPW;
+      const bool has_bias = EPI != EPI_I32 && EPI != EPI_PART && a.bias != nullptr;
 #pragma unroll
-      for (int p0 = 0; p0 < kPW; p0 += kPass) {
-        int nl[kPass * 4];  // in-range column groups for the loads
+      for (int h = 0; h < NWP; ++h) {
+        const int nh = n0 + (NWP == 2 ? (2 * wn + h) * 64 : wn * 64);
+        int nl[4];  // in-range column groups for the loads
 #pragma unroll
-        for (int j = 0; j < kPass * 4; ++j) {
-          const int n = ncol + 32 * (p0 + j / 4) + 8 * (j % 4);
-          nl[j] = n < a.N ? n : 0;
+        for (int p = 0; p < 4; ++p) {
+          const int n = nh + 16 * p + 4 * lc;
+          nl[p] = n < a.N ? n : 0;
         }
-        uint32_t sb[kPass * 4][4];
-        if constexpr (EPI == EPI_DEQ) tile_scale_bits<kPass * 4>(a.s_ch, a.s_ch_dtype, nl, sb);
-        V4 bv[kPass][4];
+        V4 bv[4];
         if (has_bias) {
 #pragma unroll
-          for (int j = 0; j < kPass * 4; ++j) bv[j / 4][j % 4] = *(const V4*)((const TO*)a.bias + nl[j]);
+          for (int p = 0; p < 4; ++p) bv[p] = *(const V4*)((const char*)a.bias + (uint32_t)(nl[p] * (int)sizeof(TO)));
         }
+        float sc[4][4];
+        if constexpr (EPI == EPI_DEQ) tile_scales<4>(a.s_ch, a.s_ch_dtype, nl, sc);
 #pragma unroll
-        for (int pp = 0; pp < kPass; ++pp)
+        for (int j = 0; j < NXP; ++j)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int p = p0 + pp;
-            const int n = ncol + 32 * p + 8 * g;
-            const bool n_ok = n < a.N;
+          for (int p = 0; p < 4; ++p) {
 #pragma unroll
-            for (int q = 0; q < kQX; ++q) {
-              const int m = mrow + 32 * q;
+            for (int q = 0; q < 2; ++q) {
               TO o[4];
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
-                if constexpr (EPI == EPI_I32) {
-                  o[i] = (TO)acc[p][q][4 * g + i];
+                if constexpr (EPI == EPI_I32 || EPI == EPI_PART) {
+                  o[i] = (TO)acc[h][j][p][q][i];
                 } else if constexpr (EPI == EPI_DEQ) {
                   // the product is rounded before the bias is added (no fused
                   // multiply-add), as in ll_dequant_splitk followed by the add
-                  const float sc = ll_scale_bits_to_f32(sb[4 * pp + g][i], a.s_ch_dtype);
-                  float v = (float)acc[p][q][4 * g + i] * st[q] * sc;
+                  float v = (float)acc[h][j][p][q][i] * st[j][q] * sc[p][i];
                   asm volatile("" : "+v"(v));
-                  if (has_bias) v += ll_to_f32(bv[pp][g][i]);
+                  if (has_bias) v += ll_to_f32(bv[p][i]);
                   o[i] = ll_from_f32<TO>(v);
                 } else {
-                  o[i] = ll_from_f32<TO>(acc[p][q][4 * g + i] +
-                                         (has_bias ? ll_to_f32(bv[pp][g][i]) : 0.f));
+                  o[i] = ll_from_f32<TO>(acc[h][j][p][q][i] + (has_bias ? ll_to_f32(bv[p][i]) : 0.f));
                 }
               }
-              const uint32_t off = (n_ok && m < a.M)
-                                       ? (uint32_t)(((int64_t)m * a.ldy + n) * (int64_t)sizeof(TO))
-                                       : kTileNoStore;
-              tile_store4<TO>(yres, off, o);
+              ep_put(16 * q + lr, 16 * p % kSegCols + 4 * lc, o);
             }
+            if (16 * (p + 1) % kSegCols == 0)
+              ep_store(el, yres, mw + 128 * j, nh + 16 * (p + 1) - kSegCols, a.N);
           }
       }
     } else {
-      // gate/up interleaved in 64-row blocks: this wave's rows 0..63 (p < 2)
-      // are gate channels c, rows 64..127 (p >= 2) the up channels c, with
-      // c = n0 / 2 + wn * 64 + 32 (p % 2) + 8g + 4(l / 32) + i; N = 2 I
+      // gate/up interleaved in 64-row blocks; this wave's channels:
+      //   2 x *: n0 / 2 + 64 wn + 16 p, gate acc[0][j][p], up acc[1][j][p]
+      //   1 x *: n0 / 2 + 32 wn + 16 p, gate acc[0][j][p], up acc[0][j][p + 2]
+      constexpr int NB = 2 * NWP;  // 16-channel blocks of this wave
       const int I = a.N / 2;
-      const int cbase = n0 / 2 + wn * 64 + 4 * lc;
-      // scales of the gate channels (groups 0..7) and the up channels (8..15)
-      uint32_t sb[16][4];
+      const int cw = n0 / 2 + wn * 16 * NB;
+      float sc[2 * NB][4];  // scales of the gate channels, then the up channels
       if constexpr (EPI == EPI_DEQ_SILU) {
-        int cl[16];
+        int cl[2 * NB];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int c = cbase + 32 * (j / 4) + 8 * (j % 4);
-          cl[j] = c < I ? c : 0;
-          cl[8 + j] = I + cl[j];
+        for (int p = 0; p < NB; ++p) {
+          const int c = cw + 16 * p + 4 * lc;
+          cl[p] = c < I ? c : 0;
+          cl[NB + p] = I + cl[p];
         }
-        tile_scale_bits<16>(a.s_ch, a.s_ch_dtype, cl, sb);
+        tile_scales<2 * NB>(a.s_ch, a.s_ch_dtype, cl, sc);
       }
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+      for (int j = 0; j < NXP; ++j)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int c = cbase + 32 * p + 8 * g;
-          const bool c_ok = c < I;
+        for (int p = 0; p < NB; ++p) {
 #pragma unroll
-          for (int q = 0; q < kQX; ++q) {
-            const int m = mrow + 32 * q;
+          for (int q = 0; q < 2; ++q) {
+            const auto ga = acc[0][j][p][q];
+            const auto ua = NWP == 2 ? acc[NWP - 1][j][p][q] : acc[0][j][(p + 2) % 4][q];
             TO o[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               float gs, us;
               if constexpr (EPI == EPI_DEQ_SILU) {
-                gs = (float)acc[p][q][4 * g + i] * st[q] *
-                     ll_scale_bits_to_f32(sb[4 * p + g][i], a.s_ch_dtype);
-                us = (float)acc[p + 2][q][4 * g + i] * st[q] *
-                     ll_scale_bits_to_f32(sb[8 + 4 * p + g][i], a.s_ch_dtype);
+                gs = (float)ga[i] * st[j][q] * sc[p][i];
+                us = (float)ua[i] * st[j][q] * sc[NB + p][i];
               } else {
-                gs = acc[p][q][4 * g + i];
-                us = acc[p + 2][q][4 * g + i];
+                gs = ga[i];
+                us = ua[i];
               }
               const float gv = ll_to_f32(ll_from_f32<TO>(gs));
               const float u = ll_to_f32(ll_from_f32<TO>(us));
               const TO sv = ll_from_f32<TO>(ll_silu_f32(gv));
               o[i] = ll_from_f32<TO>(u * ll_to_f32(sv));
             }
-            const uint32_t off = (c_ok && m < a.M)
-                                     ? (uint32_t)(((int64_t)m * a.ldy + c) * (int64_t)sizeof(TO))
-                                     : kTileNoStore;
-            tile_store4<TO>(yres, off, o);
+            ep_put(16 * q + lr, 16 * p % kSegCols + 4 * lc, o);
           }
+          if (16 * (p + 1) % kSegCols == 0)
+            ep_store(el, yres, mw + 128 * j, cw + 16 * (p + 1) - kSegCols, I);
         }
     }
   };
 
-  // Ping-pong schedule. Waves 0-3 (group A) and 4-7 (group B) hold one
-  // wave of each SIMD (the dispatcher places wave w on SIMD w % 4). Time is
-  // cut into phases separated by workgroup barriers; in phase 2g group A
-  // multiplies stage g (of this workgroup's stage sequence) from its
-  // registers while group B reads its fragments of stage g from LDS and
-  // issues its half of the copies of stage g + 4, and in phase 2g + 1 the
-  // roles swap (B multiplies stage g, A reads stage g + 1 and issues its
-  // half of stage g + 4). Each SIMD's MFMA pipe so always has one wave with
-  // a run of 16 independent MFMAs while the other wave's LDS reads and
-  // copies proceed. Ring invariants (five buffers, stage t in buffer t % 5):
-  //   * stage t lands before the barrier that ends phase 2t - 2 (A waits
-  //     vmcnt(8) at the end of its compute phase, B vmcnt(12) after
-  //     issuing), so A's reads in phase 2t - 1 and B's in phase 2t see it;
-  //   * the copies of stage t + 5 go to stage t's buffer in phases 2t + 2
-  //     and 2t + 3, after the barrier that ends B's last read of stage t
-  //     (phase 2t, closed by lgkmcnt(0)).
-  // A wave writes a finished tile's outputs in its first memory phase after
-  // the tile's last stage (A: phase 2g + 1, B: phase 2g + 2), before that
-  // phase's copies, and does not wait for the stores: the vmcnt waits of
-  // the next phases allow kStores more operations when stores were issued
-  // after the copies they wait for (a count at or below the exact one is
-  // always safe; vmcnt retires in issue order).
-  static_assert(kNst == 5 && kDmaW == 4, "the ping-pong wait counts assume 5 buffers, 4 copies");
-  static_assert(12 + kStores < 64, "vmcnt is a 6-bit counter");
+  // Ping-pong schedule. Waves 0-3 (group A) and 4-7 (group B) hold one wave
+  // of each SIMD (the dispatcher places wave w on SIMD w % 4). Time is cut
+  // into slots separated by workgroup barriers. In slot 2P group A reads the
+  // fragments of phase P and issues copies while group B multiplies phase
+  // P - 1; in slot 2P + 1 A multiplies phase P while B reads it. So each
+  // SIMD's matrix pipe has one wave with a run of MFMAs while the other
+  // wave's LDS reads and copies proceed. Ring invariants (R = kNst * kPh read
+  // phases in the ring):
+  //   * the pieces of read phase P have landed before slot 2P: each wave
+  //     issues them in its memory slot of phase P + 1 - R and waits for them
+  //     (vmcnt) before the barrier that ends slot 2P - 1, with the copies of
+  //     R - 2 later phases outstanding (wait_cnt);
+  //   * the buffer of read phase P - 1's pieces is refilled in the memory
+  //     slots of phase P (2P and 2P + 1), after the barrier that ends B's
+  //     read of them (slot 2P - 1, closed by lgkmcnt(0)).
+  // A wave writes a finished item's outputs in its first memory slot after
+  // the item's last stage, before that slot's copies, and does not wait for
+  // the stores: while the copies waited for were issued before the stores,
+  // the waits allow kStores more operations (a count at or below the exact
+  // one is always safe; vmcnt retires in issue order).
+  static_assert(G::wait_cnt(0) + kStores < 64 && G::wait_cnt(kPh - 1) + kStores < 64,
+                "vmcnt is a 6-bit counter");
+  constexpr int kAllow = kNst * kPh - 3;  // phases after an epilogue whose waits it may outlast
+  int since_ep = 64;                      // phases since this wave's last epilogue
+  auto wait_for = [&](auto qc) LL_INLINE {
+    constexpr int n = G::wait_cnt(decltype(qc)::value);
+    if (since_ep <= kAllow) tile_vm_wait<n + kStores>();
+    else tile_vm_wait<n>();
+    ++since_ep;
+  };
+  auto ph_const = [](auto f) LL_INLINE {  // calls f(integral_constant<0..kPh-1>) in order
+    f(std::integral_constant<int, 0>{});
+    if constexpr (kPh > 1) f(std::integral_constant<int, 1>{});
+  };
   const bool group_a = wave < 4;
-  // prologue: B issues its halves of stages 0..3, A of stages 0..2; stage 0
-  // lands; A reads stage 0 and issues its half of stage 3 (phase -1)
-  issue();
-  issue();
-  issue();
-  if (group_a) {
-    tile_vm_wait<8>();
-  } else {
-    issue();
-    tile_vm_wait<12>();
-  }
+  // cursor of the multiplications
+  int cur_i = i_first, cur_k, cur_ke;
+  auto cur_item = [&]() LL_INLINE {
+    const int sp = cur_i / tiles;
+    cur_k = sp * a.kps;
+    cur_ke = min(cur_k + a.kps, a.nk);
+  };
+  cur_item();
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, kPh - 1> ph_last{};
+  // prologue: every read phase of the ring but the last one (after the first
+  // X0 where it is read ahead, which both groups read before the first slot)
+  if constexpr (G::kAhead) issue_piece(std::integral_constant<int, 3>{});
+#pragma unroll
+  for (int s = 0; s < kNst; ++s)
+    ph_const([&](auto ph) LL_INLINE {
+      if (s < kNst - 1 || decltype(ph)::value < kPh - 1) issue(ph);
+    });
+  tile_vm_wait<G::wait_cnt(0)>();
   tile_barrier();
-  if (group_a) {
-    read_stage(0);
-    issue();
+  if constexpr (G::kAhead) {
+    read_x(std::integral_constant<int, 3>{}, 0, fx[2]);
+    tile_barrier();
   }
-  tile_barrier();
-  // sched_barrier keeps every instruction inside its phase (MFMAs touch no
+  int buf = 0;
+  bool more = true;
+  // sched_barrier keeps every instruction inside its slot (MFMAs touch no
   // memory, so nothing else stops the scheduler moving them across barriers)
-  int cks = 0;        // stage within its tile of the stage being multiplied
-  int last_ep = -8;   // iteration of this wave's last epilogue
+  auto stage_a = [&]() LL_INLINE {
+    const bool full = !(a.half && cur_k == a.nk - 1);
+    const bool last = cur_k + 1 == cur_ke;  // the item's last stage
+    const int nbuf = buf == kNst - 1 ? 0 : buf + 1;
+    ph_const([&](auto phc) LL_INLINE {
+      constexpr int ph = decltype(phc)::value;
+      constexpr std::integral_constant<int, (ph + 1) % kPh> nxt{};
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+      multiply(phc, full);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_for(nxt);
+      tile_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (ph == kPh - 1) {
+        if (last) {
+          epilogue(cur_i);
+          zero_acc();
+          since_ep = 0;
+        }
+      }
+      read_phase(nxt, ph == kPh - 1 ? nbuf : buf);
+      issue(phc);
+      __builtin_amdgcn_sched_barrier(0);
+      tile_barrier();
+    });
+    buf = nbuf;
+    if (!last) {
+      ++cur_k;
+    } else {
+      cur_i += g8;
+      more = cur_i < i_end;
+      if (more) cur_item();
+    }
+  };
+  int done = -1;  // group B: item whose outputs are still in the accumulators
+  auto stage_b = [&]() LL_INLINE {
+    const bool full = !(a.half && cur_k == a.nk - 1);
+    const bool last = cur_k + 1 == cur_ke;
+    ph_const([&](auto phc) LL_INLINE {
+      constexpr int ph = decltype(phc)::value;
+      constexpr std::integral_constant<int, (ph + 1) % kPh> nxt{};
+      constexpr std::integral_constant<int, (ph + kPh - 1) % kPh> prv{};
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (ph == 0) {
+        if (done >= 0) {
+          epilogue(done);
+          zero_acc();
+          since_ep = 0;
+          done = -1;
+        }
+      }
+      read_phase(phc, buf);
+      issue(prv);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_for(nxt);
+      tile_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+      multiply(phc, full);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      tile_barrier();
+    });
+    buf = buf == kNst - 1 ? 0 : buf + 1;
+    if (!last) {
+      ++cur_k;
+    } else {
+      done = cur_i;
+      cur_i += g8;
+      more = cur_i < i_end;
+      if (more) cur_item();
+    }
+  };
   if (group_a) {
-    for (int g = 0; g < total; ++g) {
-      __builtin_amdgcn_sched_barrier(0);
-      compute();                 // phase 2g: stage g
-      __builtin_amdgcn_sched_barrier(0);
-      // own copies of stage g + 1 landed; they were issued in iteration
-      // g - 3, before the stores of an epilogue in iteration g - 2 or g - 1
-      if (g - last_ep <= 2) tile_vm_wait<8 + kStores>();
-      else tile_vm_wait<8>();
-      tile_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if (cks == nk - 1) {       // phase 2g + 1
-        epilogue();
-        zero_acc();
-        last_ep = g;
-      }
-      read_stage(g + 1);
-      issue();                   // stage g + 4
-      __builtin_amdgcn_sched_barrier(0);
-      tile_barrier();
-      cks = cks == nk - 1 ? 0 : cks + 1;
-    }
+    read_phase(c0, 0);
+    issue(ph_last);
+    tile_barrier();
+    while (more) stage_a();
   } else {
-    for (int g = 0; g < total; ++g) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (g > 0 && cks == 0) {   // phase 2g: the previous tile's outputs
-        epilogue();
-        zero_acc();
-        last_ep = g;
-      }
-      read_stage(g);
-      issue();                   // stage g + 4
-      __builtin_amdgcn_sched_barrier(0);
-      // own copies of stage g + 1 landed; they were issued in iteration
-      // g - 3, before the stores of an epilogue in iteration g - 2 .. g
-      if (g - last_ep <= 2) tile_vm_wait<12 + kStores>();
-      else tile_vm_wait<12>();
-      tile_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      compute();                 // phase 2g + 1: stage g
-      __builtin_amdgcn_sched_barrier(0);
-      tile_barrier();
-      cks = cks == nk - 1 ? 0 : cks + 1;
-    }
-    epilogue();
+    tile_barrier();
+    while (more) stage_b();
+    epilogue(done);
   }
   __builtin_amdgcn_sched_barrier(0);
   tile_vm_wait<0>();
@@ -522,39 +717,95 @@ __global__ void interleave_gate_up_kernel(const u32x4* __restrict__ W, int64_t l
   out[u] = W[src * ldw16 + c];
 }
 
+// Row tiles per group of the tile order, by shape class, as measured on the
+// 3B prefill projections at M = 24,000 (group sizes 1, 2, 4 and 8, libraries
+// interleaved, best of 4 rounds): wide outputs (gate/up, 86 column tiles)
+// 4 (1788 us against 1813 with 2 and 1886-1898 with 1 or 8); long K
+// (down_proj, 172 stages) 1 (916 against 953 with 2); the narrow short-K
+// shapes (qkv, o_proj) level at every size (2).
+int tile_group_m(int64_t tiles_n, int64_t nk) {
+  if (tiles_n >= 32) return 4;
+  if (nk >= 64) return 1;
+  return 2;
+}
+
+struct TilePlan {
+  int geo;     // 0: 256 x 256, 1: 256 x 128, 2: 128 x 128
+  int splits;  // k splits
+  int kps;     // stages per split
+};
+
+// Tile geometry and k splits by a cost in us, fitted to a sweep of every
+// geometry and split count over M 96 .. 24000 at the 3B and 1.5B projections
+// (cold weights): a stage costs 1.15 us with few workgroups and 1.5 with all
+// CUs busy (256 x 256), 0.87 .. 1.0 (256 x 128), 0.55 (128 x 128); an item
+// 6, 2 and 3.7 us of fill and stores; the reduction of splits one more launch
+// and the partials' bytes both ways. So large outputs take 256 x 256 tiles
+// (M = 24,000, gate/up: 1736 us against 2244 and 2702), outputs of few tiles
+// smaller ones and splits (333 x 2048, K = 11008: 33 us with 128 x 128 tiles
+// in 5 splits, 98 unsplit, 197 as 16 tiles of 256 x 256), and what lies
+// between follows the rounds its tiles take (600 x 22016: 71 us in two
+// rounds of 256 x 128, 97 in two of 256 x 256).
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t nk, int64_t max_splits, int cus) {
+  static const int tn[3] = {256, 256, 128}, tm[3] = {256, 128, 128};
+  static const double stage_us[3] = {1.15, 0.87, 0.55}, busy_us[3] = {0.35, 0.13, 0.0};
+  static const double item_us[3] = {6.0, 2.0, 3.7};
+  TilePlan best = {0, 1, (int)nk};
+  double best_us = 1e30;
+  for (int g = 0; g < 3; ++g) {
+    const int64_t tiles = (int64_t)ll_cdiv(M, tm[g]) * ll_cdiv(N, tn[g]);
+    for (int64_t sp = 1; sp <= max_splits; ++sp) {
+      if (sp > 1 && (sp * kMinSplitStages > nk || tiles * sp > cus)) break;
+      const int64_t kps = ll_cdiv(nk, sp);
+      if (ll_cdiv(nk, kps) != sp) continue;  // an empty last split
+      const int64_t items = tiles * sp, per = ll_cdiv(items, 8);
+      const int64_t g8 = std::min<int64_t>(per, std::max(1, cus / 8));
+      const double busy = std::min(1.0, (double)items / cus);
+      const double us = (double)ll_cdiv(per, g8) * (kps * (stage_us[g] + busy_us[g] * busy) + item_us[g]) +
+                        (sp > 1 ? 4.5 + (double)sp * M * N * 8 / 5.5e6 : 0.0);
+      if (us < best_us) {
+        best_us = us;
+        best = {g, (int)sp, (int)kps};
+      }
+    }
+  }
+  return best;
+}
+
 // The kernel addresses its copy sources with 32-bit row offsets and its
 // stores with 31-bit buffer offsets: the weight must span less than 4 GiB
 // (checked by the entry points), and the activation and output rows are
 // launched in chunks whose spans fit (and whose stage count per workgroup
 // fits an int).
-template <typename T, typename TO, int EPI>
-int launch_tiles(const TileArgs& a0, hipStream_t stream) {
-  int cus = 0;
-  const int rc = ll_device_cus(&cus);
-  if (rc != LL_OK) return rc;
+template <typename T, typename TO, int EPI, typename G>
+int launch_geo(const TileArgs& a0, const TilePlan& plan, int cus, hipStream_t stream) {
   const int64_t yrow_b = a0.ldy * (int64_t)sizeof(TO);
-  const int64_t tiles_n = ll_cdiv(a0.N, kT), nk = a0.K_b / kRB;
+  const int64_t ny = EPI == EPI_SILU || EPI == EPI_DEQ_SILU ? a0.N / 2 : a0.N;
+  const int64_t tiles_n = ll_cdiv(a0.N, G::TN);
   const int64_t rows_x = (((int64_t)1 << 32) - 2 * kRB) / a0.ldx_b;
   const int64_t rows_y = (((int64_t)1 << 31) - 1) / yrow_b;
-  const int64_t rows_s = ((int64_t)INT32_MAX / nk) * 8 / tiles_n * kT;
+  const int64_t rows_s = ((int64_t)INT32_MAX / a0.nk) * 8 / (tiles_n * plan.splits) * G::TM;
   const int64_t max_rows = std::min(rows_x, std::min(rows_y, rows_s));
   LL_CHECK_ARG(max_rows >= 1, "gemm tiles: output rows or K too large for one launch");
   const int64_t chunk =
-      max_rows >= a0.M ? a0.M : (max_rows >= kT ? (max_rows / kT) * kT : max_rows);
+      max_rows >= a0.M ? a0.M : (max_rows >= G::TM ? (max_rows / G::TM) * G::TM : max_rows);
   for (int64_t mo = 0; mo < a0.M; mo += chunk) {
     TileArgs a = a0;
     a.X += mo * a0.ldx_b;
     a.Y = (char*)a0.Y + mo * yrow_b;
     if (a0.s_tok != nullptr) a.s_tok = a0.s_tok + mo;
     a.M = (int)(a0.M - mo < chunk ? a0.M - mo : chunk);
-    a.y_bytes = (int)((a.M - 1) * yrow_b + a.N * (int64_t)sizeof(TO));
-    a.tiles_m = ll_cdiv(a.M, kT);
+    a.y_bytes = (int)((a.M - 1) * yrow_b + ny * (int64_t)sizeof(TO));
+    a.wide = yrow_b % 16 == 0 && (uintptr_t)a0.Y % 16 == 0 && (ny * (int64_t)sizeof(TO)) % 16 == 0;
+    a.tiles_m = ll_cdiv(a.M, G::TM);
     a.tiles_n = (int)tiles_n;
-    a.group_m = tile_group_m(tiles_n, nk);
-    const int64_t per = ((int64_t)a.tiles_m * a.tiles_n + 7) / 8;
+    a.splits = plan.splits;
+    a.kps = plan.kps;
+    a.group_m = tile_group_m(tiles_n, a.nk);
+    const int64_t per = ((int64_t)a.tiles_m * a.tiles_n * a.splits + 7) / 8;
     const int64_t grid = 8 * std::min<int64_t>(per, std::max(1, cus / 8));
-    hipLaunchKernelGGL((gemm_tile_kernel<T, TO, EPI>), dim3((unsigned)grid), dim3(kThreads),
-                       (size_t)kNst * kStageB, stream, a);
+    hipLaunchKernelGGL((gemm_tile_kernel<T, TO, EPI, G>), dim3((unsigned)grid), dim3(kThreads),
+                       G::kLds, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
       ll_set_error("HIP launch failed: %s", hipGetErrorString(e));
@@ -564,15 +815,93 @@ int launch_tiles(const TileArgs& a0, hipStream_t stream) {
   return LL_OK;
 }
 
+template <typename T, typename TO, int EPI>
+int launch_plan(const TileArgs& a, const TilePlan& plan, int cus, hipStream_t stream) {
+  if (plan.geo == 0) return launch_geo<T, TO, EPI, TileGeo<2, 2>>(a, plan, cus, stream);
+  if (plan.geo == 1) return launch_geo<T, TO, EPI, TileGeo<2, 1>>(a, plan, cus, stream);
+  return launch_geo<T, TO, EPI, TileGeo<1, 1>>(a, plan, cus, stream);
+}
+
+// one k split, outputs in their final form
+template <typename T, typename TO, int EPI>
+int launch_tiles(const TileArgs& a, hipStream_t stream) {
+  int cus = 0;
+  const int rc = ll_device_cus(&cus);
+  if (rc != LL_OK) return rc;
+  return launch_plan<T, TO, EPI>(a, plan_tiles(a.M, a.N, a.nk, 1, cus), cus, stream);
+}
+
+// Sum of the k splits' partials [splits][M][N], in split order, finished as
+// the tile epilogue finishes its sums: fp32 (+ bias), or int32 dequantised.
+// 4 columns per thread.
+template <typename TP, typename TO>
+__global__ __launch_bounds__(256) void tile_reduce_kernel(const TP* __restrict__ part, int splits,
+                                                          const void* __restrict__ bias,
+                                                          const float* __restrict__ s_tok,
+                                                          const void* __restrict__ s_ch,
+                                                          int s_ch_dtype, TO* __restrict__ Y,
+                                                          int64_t ldy, int M, int N) {
+  typedef TO V4 __attribute__((ext_vector_type(4)));
+  const int q = N / 4;
+  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int m = (int)(gid / q);
+  if (m >= M) return;
+  const int n = (int)(gid - (int64_t)m * q) * 4;
+  const int64_t idx = (int64_t)m * N + n, ss = (int64_t)M * N;
+  V4 o;
+  if constexpr (__is_same(TP, float)) {
+    const f32x4 v = ll_sum_splits4(part, splits, ss, idx);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = ll_from_f32<TO>(v[e] + (bias != nullptr ? ll_to_f32(((const TO*)bias)[n + e]) : 0.f));
+  } else {
+    const i32x4 v = ll_sum_splits4_i32(part, splits, ss, idx);
+    const float st = s_tok[m];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float x = (float)v[e] * st * ll_load_scale(s_ch, s_ch_dtype, n + e);
+      asm volatile("" : "+v"(x));
+      if (bias != nullptr) x += ll_to_f32(((const TO*)bias)[n + e]);
+      o[e] = ll_from_f32<TO>(x);
+    }
+  }
+  *(V4*)(Y + (int64_t)m * ldy + n) = o;
+}
+
+// Product with the K of few output tiles split over the CUs: partial sums in
+// the workspace and a reduction, where the plan splits and the workspace
+// holds them; else one split.
+template <typename T, typename TO, int EPI>
+int launch_tiles_ws(const TileArgs& a, void* ws, int64_t ws_bytes, hipStream_t stream) {
+  typedef typename std::conditional<__is_same(T, int8_t), int32_t, float>::type TP;
+  int cus = 0;
+  const int rc = ll_device_cus(&cus);
+  if (rc != LL_OK) return rc;
+  const int64_t split_b = (int64_t)a.M * a.N * 4;
+  const int64_t room = ws != nullptr && (uintptr_t)ws % 16 == 0 ? ws_bytes / split_b : 0;
+  const TilePlan plan = plan_tiles(a.M, a.N, a.nk, std::max<int64_t>(1, room), cus);
+  if (plan.splits == 1) return launch_plan<T, TO, EPI>(a, plan, cus, stream);
+  TileArgs pa = a;
+  pa.Y = ws;
+  pa.ldy = a.N;
+  pa.split_b = split_b;
+  const int prc = launch_plan<T, TP, __is_same(T, int8_t) ? EPI_I32 : EPI_PART>(pa, plan, cus, stream);
+  if (prc != LL_OK) return prc;
+  hipLaunchKernelGGL((tile_reduce_kernel<TP, TO>), dim3((unsigned)ll_cdiv((int64_t)a.M * (a.N / 4), 256)),
+                     dim3(256), 0, stream, (const TP*)ws, plan.splits, a.bias, a.s_tok, a.s_ch,
+                     a.s_ch_dtype, (TO*)a.Y, a.ldy, a.M, a.N);
+  LL_RETURN_LAUNCH();
+}
+
 // ldx, ldw in elements of es bytes; ldy in elements of Y, whose rows hold
 // ny outputs (N, or N / 2 for the gate/up epilogues).
 int check_tile_args(const char* name, const void* X, int64_t ldx, const void* W, int64_t ldw,
                     const void* Y, int64_t ldy, int64_t ny, int64_t M, int64_t N, int64_t K_b,
                     int64_t es) {
   LL_CHECK_ARG(X && W && Y, "%s: null pointer", name);
-  LL_CHECK_ARG(M > 0 && N > 0 && N % 4 == 0 && K_b > 0 && K_b % kRB == 0,
+  LL_CHECK_ARG(M > 0 && N > 0 && N % 4 == 0 && K_b > 0 && K_b % kKUnit == 0,
                "%s: needs M > 0, N %% 4 == 0 and K a multiple of %lld (M=%lld N=%lld K=%lld)", name,
-               (long long)(kRB / es), (long long)M, (long long)N, (long long)(K_b / es));
+               (long long)(kKUnit / es), (long long)M, (long long)N, (long long)(K_b / es));
   LL_CHECK_ARG(ldx * es >= K_b && ldw * es >= K_b && ldy >= ny,
                "%s: row strides shorter than the rows (ldx=%lld ldw=%lld K=%lld, ldy=%lld for "
                "%lld outputs per row)",
@@ -592,7 +921,9 @@ TileArgs make_args(const void* X, int64_t ldx_b, const void* W, int64_t ldw_b, i
   TileArgs a = {};
   a.X = (const char*)X; a.ldx_b = ldx_b;
   a.W = (const char*)W; a.ldw_b = ldw_b;
-  a.M = (int)M; a.N = (int)N; a.K_b = (int)K_b;
+  a.M = (int)M; a.N = (int)N;
+  a.nk = a.kps = ll_cdiv(K_b, kRB);
+  a.half = K_b % kRB != 0;
   a.Y = Y; a.ldy = ldy;
   return a;
 }
@@ -621,12 +952,12 @@ int ll_device_cus(int* cus_out) {
 
 extern "C" int ll_gemm_tiled_supported(int64_t M, int64_t N, int64_t K, int dtype) {
   if (dtype != LL_BF16 && dtype != LL_F16) return 0;
-  return M > 0 && N > 0 && N % 4 == 0 && K > 0 && (K * 2) % kRB == 0;
+  return M > 0 && N > 0 && N % 4 == 0 && K > 0 && (K * 2) % kKUnit == 0;
 }
 
-extern "C" int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t ldw,
-                             const void* bias, void* Y, int64_t ldy, int64_t M, int64_t N,
-                             int64_t K, int dtype, hipStream_t stream) {
+int ll_gemm_tiled_ws(const void* X, int64_t ldx, const void* W, int64_t ldw, const void* bias,
+                     void* Y, int64_t ldy, int64_t M, int64_t N, int64_t K, int dtype, void* ws,
+                     int64_t ws_bytes, hipStream_t stream) {
   LL_CHECK_ARG(dtype == LL_BF16 || dtype == LL_F16, "ll_gemm_tiled: bf16 or fp16 only");
   const int rc = check_tile_args("ll_gemm_tiled", X, ldx, W, ldw, Y, ldy, N, M, N, K * 2, 2);
   if (rc != LL_OK) return rc;
@@ -634,8 +965,23 @@ extern "C" int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t 
   LL_CHECK_ARG(((uintptr_t)bias) % 8 == 0, "ll_gemm_tiled: bias must be 8 B aligned");
   TileArgs a = make_args(X, ldx * 2, W, ldw * 2, M, N, K * 2, Y, ldy);
   a.bias = bias;
-  if (dtype == LL_BF16) return launch_tiles<__bf16, __bf16, EPI_STORE>(a, stream);
-  return launch_tiles<_Float16, _Float16, EPI_STORE>(a, stream);
+  if (dtype == LL_BF16) return launch_tiles_ws<__bf16, __bf16, EPI_STORE>(a, ws, ws_bytes, stream);
+  return launch_tiles_ws<_Float16, _Float16, EPI_STORE>(a, ws, ws_bytes, stream);
+}
+
+extern "C" int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t ldw,
+                             const void* bias, void* Y, int64_t ldy, int64_t M, int64_t N,
+                             int64_t K, int dtype, hipStream_t stream) {
+  return ll_gemm_tiled_ws(X, ldx, W, ldw, bias, Y, ldy, M, N, K, dtype, nullptr, 0, stream);
+}
+
+extern "C" int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K,
+                                                int64_t elem_bytes) {
+  if (M <= 64 || N <= 0 || N % 4 != 0 || K <= 0 || (elem_bytes != 1 && elem_bytes != 2) ||
+      (K * elem_bytes) % kKUnit != 0)
+    return 0;
+  const TilePlan p = plan_tiles(M, N, ll_cdiv(K * elem_bytes, kRB), kPlanCus, kPlanCus);
+  return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
 }
 
 extern "C" int ll_gemm_interleave_gate_up(const void* W, int64_t ldw, int64_t I, int64_t K,
@@ -666,10 +1012,11 @@ extern "C" int ll_gemm_gate_up_silu_tiled(const void* X, int64_t ldx, const void
   return launch_tiles<_Float16, _Float16, EPI_SILU>(a, stream);
 }
 
-extern "C" int ll_gemm_i8_tiled(const int8_t* Xq, int64_t ldx, const float* s_tok,
+extern "C" int ll_gemm_i8_tiled_ws(const int8_t* Xq, int64_t ldx, const float* s_tok,
                                 const int8_t* Wq, int64_t ldw, const void* s_ch, int s_ch_dtype,
                                 const void* bias, void* Y, int64_t ldy, int64_t M, int64_t N,
-                                int64_t K, int out_dtype, hipStream_t stream) {
+                                int64_t K, int out_dtype, void* workspace,
+                                int64_t workspace_bytes, hipStream_t stream) {
   const int rc = check_tile_args("ll_gemm_i8_tiled", Xq, ldx, Wq, ldw, Y, ldy, N, M, N, K, 1);
   if (rc != LL_OK) return rc;
   LL_CHECK_ARG(out_dtype == LL_BF16 || out_dtype == LL_F16 || out_dtype == LL_F32,
@@ -683,9 +1030,17 @@ extern "C" int ll_gemm_i8_tiled(const int8_t* Xq, int64_t ldx, const float* s_to
   LL_CHECK_ARG(((uintptr_t)bias) % 8 == 0, "ll_gemm_i8_tiled: bias must be 8 B aligned");
   TileArgs a = make_args(Xq, ldx, Wq, ldw, M, N, K, Y, ldy);
   a.bias = bias; a.s_tok = s_tok; a.s_ch = s_ch; a.s_ch_dtype = s_ch_dtype;
-  if (out_dtype == LL_BF16) return launch_tiles<int8_t, __bf16, EPI_DEQ>(a, stream);
-  if (out_dtype == LL_F16) return launch_tiles<int8_t, _Float16, EPI_DEQ>(a, stream);
-  return launch_tiles<int8_t, float, EPI_DEQ>(a, stream);
+  if (out_dtype == LL_BF16) return launch_tiles_ws<int8_t, __bf16, EPI_DEQ>(a, workspace, workspace_bytes, stream);
+  if (out_dtype == LL_F16) return launch_tiles_ws<int8_t, _Float16, EPI_DEQ>(a, workspace, workspace_bytes, stream);
+  return launch_tiles_ws<int8_t, float, EPI_DEQ>(a, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ll_gemm_i8_tiled(const int8_t* Xq, int64_t ldx, const float* s_tok,
+                                const int8_t* Wq, int64_t ldw, const void* s_ch, int s_ch_dtype,
+                                const void* bias, void* Y, int64_t ldy, int64_t M, int64_t N,
+                                int64_t K, int out_dtype, hipStream_t stream) {
+  return ll_gemm_i8_tiled_ws(Xq, ldx, s_tok, Wq, ldw, s_ch, s_ch_dtype, bias, Y, ldy, M, N, K,
+                             out_dtype, nullptr, 0, stream);
 }
 
 extern "C" int ll_gemm_i8_i32_tiled(const int8_t* Xq, int64_t ldx, const int8_t* Wq, int64_t ldw,
@@ -754,7 +1109,7 @@ extern "C" int ll_gemm_i8_i32(const int8_t* Xq, int64_t ldx, const int8_t* Wq, i
                (long long)K);
   LL_CHECK_ARG(M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX, "ll_gemm_i8_i32: shape too large");
   if (M == 0) return LL_OK;
-  const bool tile = N % 4 == 0 && K % kRB == 0 && ldx % 16 == 0 && ldw % 16 == 0 &&
+  const bool tile = N % 4 == 0 && K % kKUnit == 0 && ldx % 16 == 0 && ldw % 16 == 0 &&
                     (((uintptr_t)Xq | (uintptr_t)Wq) % 16) == 0 && ldy % 4 == 0 &&
                     ((uintptr_t)Y) % 16 == 0;
   if (tile) return ll_gemm_i8_i32_tiled(Xq, ldx, Wq, ldw, Y, ldy, M, N, K, stream);

@@ -59,6 +59,12 @@ int ll_decode_spin_setting();
 // persistent grids hold one workgroup per CU, each looping over its work.
 int ll_device_cus(int* cus_out);
 
+// ll_gemm_tiled with a workspace for the partial sums of k splits
+// (ll_gemm_tiles_workspace_size; too small or null: one split) (gemm_tiles.hip).
+int ll_gemm_tiled_ws(const void* X, int64_t ldx, const void* W, int64_t ldw, const void* bias,
+                     void* Y, int64_t ldy, int64_t M, int64_t N, int64_t K, int dtype, void* ws,
+                     int64_t ws_bytes, hipStream_t stream);
+
 // Second pass of the first-index argmax over per-row partials [M][nparts]
 // written by another kernel (elementwise.hip).
 int ll_argmax_finish(const float* pval, const int* pidx, int64_t M, int64_t nparts, int64_t* out,

@@ -78,6 +78,19 @@ def workspace(device: torch.device, name: str, nbytes: int) -> torch.Tensor:
     return buf
 
 
+def optional_workspace(device: torch.device, name: str, nbytes: int):
+    """(pointer, bytes) of a workspace the callee can do without: (None, 0)
+    for no bytes; while a graph is captured, the buffer as it stands (nothing
+    is allocated inside a capture)."""
+    if nbytes <= 0:
+        return None, 0
+    if torch.cuda.is_current_stream_capturing():
+        buf = _WS.get(_ws_key(device, name))
+        return (None, 0) if buf is None else (buf.data_ptr(), buf.numel())
+    buf = workspace(device, name, nbytes)
+    return buf.data_ptr(), buf.numel()
+
+
 def reserve_workspace(device: torch.device, name: str, nbytes: int) -> None:
     workspace(device, name, nbytes)
 
@@ -340,11 +353,16 @@ def gemm(x, w, bias=None, out=None):
     if out is None:
         out = torch.empty((M, N), dtype=x.dtype, device=x.device)
     assert out.shape == (M, N) and out.stride(1) == 1
-    nbytes = _L.ll_gemm_workspace_size(M, N, K)
     ws_ptr, ws_n = (None, 0)
-    if nbytes > 0:
-        ws = workspace(x.device, "gemm", nbytes)
-        ws_ptr, ws_n = ws.data_ptr(), ws.numel()
+    if M > 64:
+        if x.dtype != torch.float32:
+            ws_ptr, ws_n = optional_workspace(x.device, "gemm",
+                                              _L.ll_gemm_tiles_workspace_size(M, N, K, 2))
+    else:
+        nbytes = _L.ll_gemm_workspace_size(M, N, K)
+        if nbytes > 0:
+            ws = workspace(x.device, "gemm", nbytes)
+            ws_ptr, ws_n = ws.data_ptr(), ws.numel()
     rc = _L.ll_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                     bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
                     M, N, K, dtype_code(x), ws_ptr, ws_n, _stream(x))
@@ -353,7 +371,7 @@ def gemm(x, w, bias=None, out=None):
 
 
 def gemm_tiled(x, w, bias=None, out=None):
-    """out[M, N] = x @ w^T (+ bias) on the 256 x 256 MFMA tile kernel (prefill)."""
+    """out[M, N] = x @ w^T (+ bias) on the MFMA tile kernel, in one k split (prefill)."""
     _dev(x, w, bias, out)
     M, K = x.shape
     N = w.shape[0]
@@ -413,11 +431,14 @@ def gemm_i8_tiled(xq, s_tok, wq, s_ch, bias=None, out_dtype=torch.bfloat16, out=
     assert s_tok.dtype == torch.float32 and s_ch.numel() == N
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=xq.device)
-    rc = _L.ll_gemm_i8_tiled(xq.data_ptr(), xq.stride(0), s_tok.data_ptr(), wq.data_ptr(),
-                             wq.stride(0), s_ch.data_ptr(), dtype_code(s_ch),
-                             bias.data_ptr() if bias is not None else None, out.data_ptr(),
-                             out.stride(0), M, N, K, dtype_code(out), _stream(xq))
-    _lib.check(rc, "ll_gemm_i8_tiled")
+    ws_ptr, ws_n = optional_workspace(xq.device, "gemm",
+                                      _L.ll_gemm_tiles_workspace_size(M, N, K, 1))
+    rc = _L.ll_gemm_i8_tiled_ws(xq.data_ptr(), xq.stride(0), s_tok.data_ptr(), wq.data_ptr(),
+                                wq.stride(0), s_ch.data_ptr(), dtype_code(s_ch),
+                                bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                                out.stride(0), M, N, K, dtype_code(out), ws_ptr, ws_n,
+                                _stream(xq))
+    _lib.check(rc, "ll_gemm_i8_tiled_ws")
     return out
 
 
