@@ -28,12 +28,15 @@
 //     run on one XCD) while it merges its own waves: no ticket, and no wait
 //     for stores to be acknowledged, on the way to the output (a device-scope
 //     version was measured slower than a second launch). The quantising
-//     variant (one sequence's heads span units on different XCDs) merges in
-//     the last workgroup of the sequence to take a ticket, and batches
-//     beyond kMergeUnits units in a second kernel.
+//     variant (a row holds all of a sequence's units) merges in the last
+//     workgroup of the sequence to take a ticket; more splits than a
+//     workgroup merges at once, a few long sequences (whose splits then lie
+//     on all XCDs, choose_splits) and batches beyond kMergeUnits units merge
+//     in a second kernel.
 // A generic VALU path covers fp32 and head dims other than 64/128.
 #include "ll_common.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -103,13 +106,14 @@ struct DecodeArgs {
   void* out; int64_t o_sb, o_sh;
   int B, H, KVH, G;
   int nsplit;
+  int spread;         // 1: the splits of a unit lie on all XCDs (map_block)
   int units;          // B * KVH
   int max_len;        // tokens beyond it are ignored (as the reference's grid does)
   int slots_cap;      // slot entries the LDS slot table holds (>= tiles per split * 16)
   float scale_log2;   // sm_scale * log2(e)
   float* part_acc;    // [B*H*nsplit, D] unnormalised partial outputs
   float* part_ml;     // [B*H*nsplit, 2] running max (log2 domain) and sum
-  unsigned* merge_cnt;  // [units] split tickets (zero between calls), or null: separate combine
+  unsigned* merge_cnt;  // [B] split tickets (zero between calls), or null: separate combine
   int unit_spin;        // polls before the per-unit merge gives up (0: kUnitMergeSpin)
   int unit_never;       // test mode: the per-unit merge never sees its words (gives up)
   uint32_t* err;        // set to 1 when the per-unit merge gives up, or null
@@ -279,8 +283,18 @@ __device__ __forceinline__ void clear_bh(const DecodeArgs& a, int bh, int lane) 
 // (the round-robin continues from the previous launch, so r varies), and
 // every workgroup of one sequence (all its KV heads and splits) is given an
 // index of the same residue, so they all run on one XCD and share its L2.
-__device__ __forceinline__ void map_block(int bid, int KVH, int nsplit, int& b, int& kvh,
-                                          int& split) {
+// Spread (the merge is then a kernel of its own, which needs no such
+// premise): (unit, split) in index order over all XCDs, a unit's splits
+// apart, so that a few long sequences use every XCD.
+__device__ __forceinline__ void map_block(int bid, int KVH, int nsplit, int units, bool spread,
+                                          int& b, int& kvh, int& split) {
+  if (spread) {
+    split = bid / units;
+    const int u = bid - split * units;
+    b = u / KVH;
+    kvh = u - b * KVH;
+    return;
+  }
   const int xcd = bid & 7, slot = bid >> 3;
   const int per_seq = KVH * nsplit;
   const int k = slot / per_seq, r = slot - k * per_seq;
@@ -416,7 +430,7 @@ __device__ __forceinline__ void unit_merge_tail(const DecodeArgs& a, bool item, 
 // The split stage, for both kernels below. p_len .. idx64 are the fields of
 // the first loads (lengths, request rows, positions, new slots, the grid
 // geometry); idx64: bit 0 lengths, bit 1 request rows, bit 2 positions are
-// int64.
+// int64; bit 3 the spread block mapping.
 template <typename T, int D, int MODE>
 __device__ __forceinline__ void decode_attn_split_stage(
     const int32_t* __restrict__ p_len, const int32_t* __restrict__ p_rid,
@@ -432,9 +446,8 @@ __device__ __forceinline__ void decode_attn_split_stage(
   int32_t* s_slots = (int32_t*)(smem + TG::MAIN_B);
 
   int b, kvh, split;
-  map_block(blockIdx.x, KVH, nsplit, b, kvh, split);
+  map_block(blockIdx.x, KVH, nsplit, B * KVH, (idx64 & 8) != 0, b, kvh, split);
   if (b >= B) return;
-  const int unit = b * KVH + kvh;
   // sequence length and request row (and with ROPE the position and the new
   // slot), all loads in flight together and before anything that reads the
   // argument block (the low word of an int64 entry is the value: lengths,
@@ -732,7 +745,7 @@ __device__ __forceinline__ void decode_attn_split_stage(
   // Per-unit merge (several splits, rows not quantised): split nsplit - 1 of
   // every (sequence, KV head) merges the others' partials (unit_merge_tail).
   const bool whole_row = a.qout != nullptr;
-  const bool unit_merge = a.merge_cnt != nullptr && !whole_row && a.nsplit <= kUnitMergeSplits;
+  const bool unit_merge = a.merge_cnt != nullptr && !whole_row;
 
   // four consecutive d of one head per thread (G * D / 4 <= kWaves * 64)
   constexpr int DQ = D / 4;
@@ -799,32 +812,19 @@ __device__ __forceinline__ void decode_attn_split_stage(
   if (unit_merge) return;
 
   __shared__ unsigned s_ticket;
-  // ---- more splits than the per-unit merge holds, or quantised rows: the
-  // last split of the unit (or, with quantised rows, the last workgroup of the
-  // sequence, which merges all its heads and quantises the row) merges after
+  // ---- quantised rows: the last workgroup of the sequence merges all its
+  // heads and quantises the row after
   // every partial store has been acknowledged by the XCD's L2 (the vector L1
   // is write-through) and drops its own L1 lines before reading them.
-  const unsigned last = (unsigned)((whole_row ? a.KVH : 1) * a.nsplit - 1);
+  const unsigned last = (unsigned)(a.KVH * a.nsplit - 1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0)
-    s_ticket = __builtin_amdgcn_atomic_inc32(a.merge_cnt + (whole_row ? b : unit), last,
+    s_ticket = __builtin_amdgcn_atomic_inc32(a.merge_cnt + b, last,
                                              __ATOMIC_RELAXED, "agent");
   __syncthreads();
   if (s_ticket != last) return;
   asm volatile("buffer_inv sc0" ::: "memory");
-  if (!whole_row) {
-    for (int gg = wave; gg < G; gg += kWaves) {
-      float o[D / 64];
-      const int bh = b * a.H + kvh * G + gg;
-      combine_bh<D>(a, bh, lane, o);
-      clear_bh<D>(a, bh, lane);
-      T* op = (T*)a.out + (int64_t)b * a.o_sb + (int64_t)(kvh * G + gg) * a.o_sh;
-#pragma unroll
-      for (int q = 0; q < D / 64; ++q) op[lane + 64 * q] = ll_from_f32<T>(o[q]);
-    }
-    return;
-  }
   // the stored row is kept in LDS (the tile rings are idle) for the codes:
   // by ll_quant_per_token's rule, or with the calibrated scale *a.qstatic
   float* row = (float*)smem;
@@ -881,15 +881,15 @@ template <typename T, int D, int MODE>
 __global__ __launch_bounds__(kWaves * 64) void decode_attn_rope_kernel(DecodeArgs a) {
   asm volatile("" ::"s"(a.seq_len), "s"(a.req_idx), "s"(a.len64), "s"(a.req64), "s"(a.pos),
                "s"(a.pos64), "s"(a.new_slots));  // the four data loads go out together
-  const int idx64 = (a.len64 ? 1 : 0) | (a.req64 ? 2 : 0) | (a.pos64 ? 4 : 0);
+  const int idx64 = (a.len64 ? 1 : 0) | (a.req64 ? 2 : 0) | (a.pos64 ? 4 : 0) | (a.spread ? 8 : 0);
   decode_attn_split_stage<T, D, MODE>((const int32_t*)a.seq_len, (const int32_t*)a.req_idx,
                                       (const int32_t*)a.pos, a.new_slots, a.KVH, a.nsplit, a.B,
                                       idx64, a);
 }
 
-// Separate merge kernels, for the shapes the split stage cannot merge itself
-// (more than kMergeUnits units, or a quantised row larger than the tile
-// rings): one wave per (sequence, head).
+// Separate merge kernels, for the shapes the split stage does not merge itself
+// (spread splits, more than kMergeUnits units, or a quantised row larger than
+// the tile rings): one wave per (sequence, head).
 template <typename T, int D>
 __global__ __launch_bounds__(kCombWaves * 64) void decode_attn_combine_kernel(DecodeArgs a) {
   constexpr int DPL = D / 64;
@@ -1024,7 +1024,15 @@ constexpr int kMaxSplitTokens = 4096;  // LDS slot table bound per split (16 KB)
 constexpr int kSplitCostTiles2 = 13;    // twice the cost of one more split, in 16-token tiles
 constexpr int kMaxSplitsFill = 16;      // split bound from 8 units up (head_dim 128)
 
-int choose_nsplit(int B, int KVH, int64_t max_len, int64_t head_dim) {
+constexpr int kSpreadRounds = 3;  // rounds of tiles the spread form must save
+
+int split_wg_per_cu(int64_t head_dim) {
+  const int64_t main_b = head_dim == 64 ? TileGeom<64>::MAIN_B : TileGeom<128>::MAIN_B;
+  const int n = (int)(160 * 1024 / (main_b + 8192));
+  return n > 1 ? n : 1;
+}
+
+int choose_nsplit_xcd(int B, int KVH, int64_t max_len, int64_t head_dim) {
   const int units = B * KVH;
   const int64_t tiles = (max_len + kTT - 1) / kTT;
   // At most one dispatch round of the 256 CUs (as many split-stage
@@ -1033,8 +1041,7 @@ int choose_nsplit(int B, int KVH, int64_t max_len, int64_t head_dim) {
   // Measured at 40 sequences x 2 KV heads: one workgroup of 8 waves per CU
   // beats two of 4 waves from 600 tokens up (fewer splits to merge, the same
   // bytes in flight per CU).
-  const int64_t main_b = head_dim == 64 ? TileGeom<64>::MAIN_B : TileGeom<128>::MAIN_B;
-  const int per_cu = (int)(160 * 1024 / (main_b + 8192)) > 1 ? (int)(160 * 1024 / (main_b + 8192)) : 1;
+  const int per_cu = split_wg_per_cu(head_dim);
   int ns = 256 * per_cu / units;
   const int64_t max_ns = tiles / kWaves;
   if (ns > max_ns) ns = (int)max_ns;
@@ -1069,6 +1076,45 @@ int choose_nsplit(int B, int KVH, int64_t max_len, int64_t head_dim) {
   return ns;
 }
 
+struct SplitPlan {
+  int ns;
+  bool spread;  // the units' splits over all XCDs, merged by a second kernel
+};
+
+// The split count, and whether a unit's splits stay on one XCD (whose split
+// stage merges up to kUnitMergeSplits of them itself) or are spread over all
+// (a few long sequences otherwise leave XCDs idle or give one of them several
+// rounds of workgroups) and merged by a second launch. Swept over 1-33
+// sequences of 1000-16384 tokens, us per call:
+// * more than kUnitMergeSplits splits are spread: 1 x 6001 tokens 26.1 with
+//   47 splits on one XCD, 13.3 with 16, 11.7 spread; 1 x 4096 20.8, 11.8,
+//   10.7; 3 x 12001 28 with 42, 19.6, 17.5; 4 x 8000 17.9 and 15.4; 12 x 2000
+//   17.5 and 12.5;
+// * up to that many only where a wave of the busiest CU takes at least three
+//   rounds of tiles less (about 2.5 us each, against 4.5 us for the launch);
+// * below 8 units at most 16 splits, or one per 24 tiles (1 x 8192: 12.7 with
+//   32, 13.1 with 16, 15.8 with 64; 1 x 16384: 16.0, 19.0, 17.5), and none
+//   that saves no round of tiles (1 x 1000: 8.5 with 4, 9.8 with 7).
+// No shape takes more splits than one XCD would give it (the workspace does
+// not grow).
+SplitPlan choose_splits(int B, int KVH, int64_t max_len, int64_t head_dim) {
+  int ns = choose_nsplit_xcd(B, KVH, max_len, head_dim);
+  const int units = B * KVH;
+  const int64_t tiles = (max_len + kTT - 1) / kTT;
+  const int min_ns = (int)((tiles * kTT + kMaxSplitTokens - 1) / kMaxSplitTokens);
+  auto tile_rounds = [&](int n) { return ll_cdiv((tiles + n - 1) / n, kWaves); };
+  if (units < 8 && ns > 1) {
+    ns = std::max(min_ns, std::min(ns, std::max(16, (int)(tiles / 24))));
+    ns = std::max(min_ns, ll_cdiv(tiles, kWaves * tile_rounds(ns)));
+  }
+  if (ns > kUnitMergeSplits) return {ns, true};
+  const int per_cu = split_wg_per_cu(head_dim);
+  const int64_t xcd_wgs = (int64_t)((B + 7) / 8) * KVH * ns;
+  const int saved = (ll_cdiv(xcd_wgs, 32 * per_cu) - ll_cdiv((int64_t)units * ns, 256 * per_cu)) *
+                    tile_rounds(ns);
+  return {ns, ns > 1 && saved >= kSpreadRounds};
+}
+
 int64_t align256(int64_t x) { return ((x + 255) / 256) * 256; }
 
 
@@ -1076,7 +1122,7 @@ int64_t align256(int64_t x) { return ((x + 255) / 256) * 256; }
 template <int D, int MODE>
 void launch_split_stage(const DecodeArgs& a, int dtype, unsigned grid, size_t lds,
                         hipStream_t stream) {
-  const int idx64 = (a.len64 ? 1 : 0) | (a.req64 ? 2 : 0) | (a.pos64 ? 4 : 0);
+  const int idx64 = (a.len64 ? 1 : 0) | (a.req64 ? 2 : 0) | (a.pos64 ? 4 : 0) | (a.spread ? 8 : 0);
   const int32_t* p_len = (const int32_t*)a.seq_len;
   const int32_t* p_rid = (const int32_t*)a.req_idx;
   if constexpr (MODE == 0) {
@@ -1134,7 +1180,7 @@ std::atomic<int> g_same_launch_merge{1};
 
 int64_t workspace_bytes_for(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
                             int64_t max_len) {
-  const int ns = choose_nsplit((int)batch, (int)kv_heads, max_len, head_dim);
+  const int ns = choose_splits((int)batch, (int)kv_heads, max_len, head_dim).ns;
   if (ns <= 1) return 0;
   const int64_t parts = batch * q_heads * ns;
   return kTicketBytes                      // split tickets
@@ -1147,7 +1193,9 @@ int64_t workspace_bytes_for(int64_t batch, int64_t q_heads, int64_t kv_heads, in
 // every field but the split geometry and the workspace pointers set.
 int launch_mfma(DecodeArgs& a, int64_t head_dim, int dtype, bool rope, int64_t max_len,
                 void* workspace, int64_t workspace_bytes, hipStream_t stream) {
-  a.nsplit = choose_nsplit(a.B, a.KVH, max_len, head_dim);
+  const SplitPlan plan = choose_splits(a.B, a.KVH, max_len, head_dim);
+  a.nsplit = plan.ns;
+  a.spread = plan.spread ? 1 : 0;
   if (a.unit_spin <= 0) a.unit_spin = kUnitMergeSpin;
   if (a.nsplit > 1) {
     const int64_t need = workspace_bytes_for(a.B, a.H, a.KVH, head_dim, max_len);
@@ -1163,7 +1211,7 @@ int launch_mfma(DecodeArgs& a, int64_t head_dim, int dtype, bool rope, int64_t m
                           : (a.B <= kMergeUnits &&
                              row_b <= (head_dim == 128 ? TileGeom<128>::MAIN_B
                                                        : TileGeom<64>::MAIN_B));
-    a.merge_cnt = (fits && g_same_launch_merge.load(std::memory_order_relaxed)) ? (unsigned*)w
+    a.merge_cnt = (fits && !plan.spread && g_same_launch_merge.load(std::memory_order_relaxed)) ? (unsigned*)w
                                                                                  : nullptr;
     w += kTicketBytes;
     const int64_t parts = (int64_t)a.B * a.H * a.nsplit;
@@ -1174,7 +1222,8 @@ int launch_mfma(DecodeArgs& a, int64_t head_dim, int dtype, bool rope, int64_t m
   const int64_t tiles = (max_len + kTT - 1) / kTT;
   a.slots_cap = (int)((tiles + a.nsplit - 1) / a.nsplit) * kTT;
   const int groups = (a.B + 7) / 8;  // sequences per XCD
-  const unsigned grid = (unsigned)(groups * 8 * a.KVH * a.nsplit);
+  const unsigned grid = plan.spread ? (unsigned)(a.units * a.nsplit)
+                                    : (unsigned)(groups * 8 * a.KVH * a.nsplit);
   const size_t extra = (size_t)a.slots_cap * 4 + (rope ? (size_t)(a.G + 2) * head_dim * 2 : 0);
   const int mode = !rope ? 0 : (!a.qkv.i32 && a.qkv.splits <= kRopeF32Splits) ? 1 : 2;
   if (head_dim == 128) {
@@ -1223,7 +1272,7 @@ extern "C" int ll_decode_attention_xcc_probe(int64_t batch, int64_t q_heads, int
   LL_CHECK_ARG(out != nullptr && batch > 0 && kv_heads > 0 && q_heads % kv_heads == 0 &&
                    (head_dim == 64 || head_dim == 128) && max_len_in_batch > 0,
                "ll_decode_attention_xcc_probe: bad arguments");
-  const int nsplit = choose_nsplit((int)batch, (int)kv_heads, max_len_in_batch, head_dim);
+  const int nsplit = choose_splits((int)batch, (int)kv_heads, max_len_in_batch, head_dim).ns;
   const int groups = (int)((batch + 7) / 8);
   const int64_t grid = (int64_t)groups * 8 * kv_heads * nsplit;
   LL_CHECK_ARG(out_len >= grid, "ll_decode_attention_xcc_probe: out holds %lld of %lld entries",
@@ -1249,7 +1298,7 @@ extern "C" int ll_decode_attention_set_same_launch_merge(int enable) {
 
 extern "C" int ll_decode_attention_split_count(int64_t batch, int64_t kv_heads, int64_t head_dim,
                                                int64_t max_len_in_batch) {
-  return choose_nsplit((int)batch, (int)kv_heads, max_len_in_batch, head_dim);
+  return choose_splits((int)batch, (int)kv_heads, max_len_in_batch, head_dim).ns;
 }
 
 extern "C" int64_t ll_decode_attention_workspace_size(int64_t batch, int64_t q_heads,
