@@ -54,44 +54,44 @@ constexpr int kKUnit = 64;     // K spans a multiple of this many bytes
 constexpr int kPlanCus = 256;   // CUs the workspace query plans for
 constexpr int kMinSplitStages = 6;  // stages a k split holds at least
 constexpr int kPieceB = 128 * kRB;  // a piece: 128 rows of one operand (16 KB)
-constexpr int kWaves = 8;      // two per SIMD
-constexpr int kThreads = 64 * kWaves;
-constexpr int kDma = 2;        // 16-byte copies per lane per piece
 
 // Tile geometry: NWP pieces of 128 weight rows by NXP pieces of 128
-// activation rows (W0, W1 and X0, X1 below). The phases of stage t, in order,
-// each reading pieces from LDS and then multiplying:
-//   2 x 2 (256 x 256): W0(t) X1(t) -> W0 X0, W0 X1; W1(t) X0(t + 1) -> W1 X0, W1 X1
-//   2 x 1 (256 x 128): W0(t) X0(t) -> W0 X0; W1(t) -> W1 X0
-//   1 x 1 (128 x 128): W0(t) X0(t) -> W0 X0
-// The 2 x 2 form reads X0 a stage ahead (two register sets, by stage parity),
-// so that both phases read 12 fragments per lane for 16 MFMAs: the time of
-// the reads and of the other group's MFMAs is the same. A piece's slot in
-// the stage buffer is its place in that order.
+// activation rows (W0, W1 and X0, X1 below).
+//
+// 256 x 256 (2 x 2): 8 waves in two groups of four that take turns (kPingPong),
+// each wave 128 x 64. The phases of stage t, in order, each reading pieces
+// from LDS and then multiplying:
+//   W0(t) X1(t) -> W0 X0, W0 X1;   W1(t) X0(t + 1) -> W1 X0, W1 X1
+// X0 is read a stage ahead, so that both phases read 12 fragments per lane
+// for 32 MFMAs: the time of the reads and of the other group's MFMAs is the
+// same. A piece's slot in the stage buffer is its place in that order.
+//
+// 256 x 128 (2 x 1, 8 waves) and 128 x 128 (1 x 1, 4 waves): 64 x 64 per wave,
+// every wave reading the next stage's fragments under its MFMAs, one barrier
+// per stage. Few workgroups run these, so what counts is the time of one
+// stage, bounded by LDS (reads and copies of 96 KB per 128 x 128 stage): 0.74
+// and 0.49 us (few workgroups), against 0.87 and 0.56 with two groups taking
+// turns on 64 x 32 per wave (128 KB, and a barrier after each turn).
 template <int NWP_, int NXP_> struct TileGeo {
   static constexpr int NWP = NWP_, NXP = NXP_;
   static constexpr int TN = 128 * NWP, TM = 128 * NXP;
   static constexpr int kPieces = NWP + NXP;
-  static constexpr bool kAhead = kPieces == 4;  // X0 is read a stage ahead
-  static constexpr int kPh = NWP;               // phases per stage
+  static constexpr bool kPingPong = kPieces == 4;
+  static constexpr int kWaves = kPingPong ? 8 : 4 * NWP;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int kDma = 16 / kWaves;      // 16-byte copies per lane per piece
+  static constexpr int NH = kPingPong ? 2 : 1;  // 64-row weight blocks per wave
   static constexpr int kStageB = kPieces * kPieceB;
   static constexpr int kNst = kPieces == 4 ? 2 : kPieces == 3 ? 3 : 4;  // stage buffers
-  static constexpr int kEpB = (160 * 1024 - kNst * kStageB) / kWaves;   // epilogue bytes per wave
+  static constexpr int kEpB = kPieces == 3 ? 2048 : 4096;               // epilogue bytes per wave
   static constexpr size_t kLds = (size_t)kNst * kStageB + (size_t)kWaves * kEpB;
+  static_assert(kLds <= 160 * 1024, "LDS");
   static constexpr bool is_w(int q) { return q == 0 || q == 2; }
   static constexpr int w_half(int q) { return q / 2; }
-  static constexpr int x_half(int q) { return kAhead && q == 1 ? 1 : 0; }
-  // pieces of phase ph: first(ph) .. last(ph)
-  static constexpr int first(int ph) { return 2 * ph; }
-  static constexpr int last(int ph) { return 2 * ph + 1 < kPieces ? 2 * ph + 1 : kPieces - 1; }
-  static constexpr int copies(int ph) { return (last(ph) - first(ph) + 1) * kDma; }
-  // copies a wave has issued after those of phase q's pieces when the pieces
-  // are about to be read (the counted wait before the read)
-  static constexpr int wait_cnt(int q) {
-    int n = 0;
-    for (int i = 1; i <= kNst * kPh - 2; ++i) n += copies((q + i) % kPh);
-    return n;
-  }
+  static constexpr int x_half(int q) { return kPingPong && q == 1 ? 1 : 0; }
+  // copies of this lane a wave may leave in flight when it waits for the next
+  // pieces to be read: two phases of two pieces, or all stages but two
+  static constexpr int kInFlight = kPingPong ? 4 * kDma : (kNst - 2) * kPieces * kDma;
 };
 
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_DEQ = 2, EPI_DEQ_SILU = 3, EPI_I32 = 4, EPI_PART = 5 };
@@ -135,6 +135,7 @@ struct TileArgs {
   const char* X; int64_t ldx_b;   // activation rows (K contiguous), row stride in bytes
   const char* W; int64_t ldw_b;   // weight rows [N][K] (EPI_SILU*: interleaved gate/up)
   int M, N;
+  int K_b;                        // K in bytes
   int nk;                         // stages of the whole K
   int kps;                        // stages per k split (the last split may have fewer)
   int half;                       // the last stage of K holds 64 bytes per row, not 128
@@ -208,11 +209,12 @@ __device__ __forceinline__ void tile_scales(const void* s, int dtype, const int 
 #define LL_INLINE __attribute__((always_inline))
 
 template <typename T, typename TO, int EPI, typename G>
-__global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
+__global__ __launch_bounds__(G::kThreads, 2) void gemm_tile_kernel(TileArgs a) {
   typedef typename TileOp<T>::V V;
   typedef typename TileOp<T>::Acc Acc;
   constexpr bool kSilu = EPI == EPI_SILU || EPI == EPI_DEQ_SILU;
-  constexpr int kPh = G::kPh, kNst = G::kNst, NWP = G::NWP, NXP = G::NXP;
+  constexpr int kNst = G::kNst, NWP = G::NWP, NH = G::NH, kWaves = G::kWaves, kDma = G::kDma;
+  constexpr bool kPP = G::kPingPong;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   // ---- work items of this workgroup: (k split, output tile), splits
@@ -229,15 +231,16 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
   if (i_first >= i_end) return;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int wn = wave & 1, wm = wave >> 1;
+  const int wn = kPP ? wave & 1 : wave >> 1, wm = kPP ? wave >> 1 : wave & 1;
 
-  // ---- copy stream: the pieces of all of this workgroup's stages in phase
-  // order, running on from one item into the next. Instruction u of this wave
-  // copies rows 8 j .. 8 j + 7 (j = 8 u + wave) of a piece; lane -> row
-  // 8 j + l / 8, LDS chunk l % 8, that is global chunk (l % 8) ^ swizzle,
-  // the same for every piece. Row i of W piece h is tile row
-  //   2 x *: (2 (i / 64) + h) * 64 + i % 64 (64-row block 2 wn + h for wave column wn);
-  //   1 x *: i, or for the SiLU forms ((i / 32) % 2) * 64 + (i / 64) * 32 + i % 32,
+  // ---- copy stream: the pieces of all of this workgroup's stages in the
+  // order they are read, running on from one item into the next. Instruction
+  // u of this wave copies rows 8 j .. 8 j + 7 (j = kWaves u + wave) of a
+  // piece; lane -> row 8 j + l / 8, LDS chunk l % 8, that is global chunk
+  // (l % 8) ^ swizzle, the same for every piece. Row i of W piece h is tile row
+  //   256 x 256:  (2 (i / 64) + h) * 64 + i % 64 (64-row block 2 wn + h of wave column wn);
+  //   the others: 128 h + i, or for the SiLU forms
+  //               128 h + ((i / 32) % 2) * 64 + (i / 64) * 32 + i % 32,
   // so that a wave holds a gate channel and its up channel.
   const int gch = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
   const uint32_t tail_adj = gch >= 4 ? 64u : 0u;  // half stage: chunks past K re-read the row's last 64 B
@@ -258,12 +261,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
     for (int q = 0; q < G::kPieces; ++q)
 #pragma unroll
       for (int u = 0; u < kDma; ++u) {
-        const int i = 8 * (8 * u + wave) + (sl >> 3);
+        const int i = 8 * (kWaves * u + wave) + (sl >> 3);
         if (G::is_w(q)) {
           int r;
-          if constexpr (NWP == 2) r = (2 * (i >> 6) + G::w_half(q)) * 64 + (i & 63);
-          else if constexpr (kSilu) r = ((i >> 5) & 1) * 64 + (i >> 6) * 32 + (i & 31);
-          else r = i;
+          if constexpr (kPP) r = (2 * (i >> 6) + G::w_half(q)) * 64 + (i & 63);
+          else if constexpr (kSilu) r = G::w_half(q) * 128 + ((i >> 5) & 1) * 64 + (i >> 6) * 32 + (i & 31);
+          else r = G::w_half(q) * 128 + i;
           soff[q][u] = row_off(min(n0 + r, a.N - 1), (uint32_t)a.ldw_b);
         } else {
           const int r = G::x_half(q) * 128 + i;
@@ -280,23 +283,23 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
     iss_ke = min(iss_k + a.kps, a.nk);
   };
   iss_item();
-  // Copies of read phase rp of the cursor's stage; the last phase moves the
-  // cursor on (before X0 where that is read a stage ahead). Past the last
-  // item every lane copies the operand's first bytes (in bounds, never read,
-  // one line), so each wave issues the same number of copies in every phase.
-  auto issue_piece = [&](auto qc) LL_INLINE {
+  // Copy u of piece q of the cursor's stage. Past the last item every lane
+  // copies the operand's first bytes (in bounds, never read, one line), so
+  // each wave issues the same number of copies in every stage.
+  auto issue_copy = [&](auto qc, int u) LL_INLINE {
     constexpr int q = decltype(qc)::value;
     const bool past = iss_i >= i_end;
     const uint32_t pmask = past ? 0u : ~0u;
     const uint32_t tadj = (a.half && iss_k == a.nk - 1) ? tail_adj : 0u;
     const int64_t kb = past ? 0 : (int64_t)iss_k * kRB;
+    uint32_t o = (soff[q][u] - tadj) & pmask;
+    asm volatile("" : "+v"(o));  // no 64-bit form of it is held through the loop
+    tile_dma16((G::is_w(q) ? a.W : a.X) + kb + o,
+               smem + iss_buf * G::kStageB + q * kPieceB + (kWaves * u + wave) * 1024);
+  };
+  auto issue_piece = [&](auto qc) LL_INLINE {
 #pragma unroll
-    for (int u = 0; u < kDma; ++u) {
-      uint32_t o = (soff[q][u] - tadj) & pmask;
-      asm volatile("" : "+v"(o));  // no 64-bit form of it is held through the loop
-      tile_dma16((G::is_w(q) ? a.W : a.X) + kb + o,
-                 smem + iss_buf * G::kStageB + q * kPieceB + (8 * u + wave) * 1024);
-    }
+    for (int u = 0; u < kDma; ++u) issue_copy(qc, u);
   };
   auto issue_next = [&]() LL_INLINE {
     iss_buf = iss_buf == kNst - 1 ? 0 : iss_buf + 1;
@@ -305,20 +308,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
       if (iss_i < i_end) iss_item();
     }
   };
-  auto issue = [&](auto rpc) LL_INLINE {
-    constexpr int rp = decltype(rpc)::value;
-    issue_piece(std::integral_constant<int, G::first(rp)>{});
-    if constexpr (rp == kPh - 1 && G::kAhead) issue_next();
-    if constexpr (G::last(rp) > G::first(rp)) issue_piece(std::integral_constant<int, G::last(rp)>{});
-    if constexpr (rp == kPh - 1 && !G::kAhead) issue_next();
-  };
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
+  constexpr std::integral_constant<int, 3> c3{};
 
-  Acc acc[NWP][NXP][4][2];
+  Acc acc[NH][2][4][2];
   auto zero_acc = [&]() LL_INLINE {
 #pragma unroll
-    for (int h = 0; h < NWP; ++h)
+    for (int h = 0; h < NH; ++h)
 #pragma unroll
-      for (int j = 0; j < NXP; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int p = 0; p < 4; ++p)
 #pragma unroll
@@ -326,74 +326,47 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
   };
   zero_acc();
 
-  // ---- fragments: of a W piece this wave's 64 rows (wn) as four 16-row
-  // blocks, of an X piece its 32 rows (wm) as two; k step ks is LDS chunks
-  // 4 ks .. 4 ks + 3 (lane l / 16). Byte offset of k step ks in a row block
-  // of a piece: one register per k step, everything else of the address is
-  // scalar or immediate (opaque, so that no other form of it takes registers
-  // through the loop).
+  // ---- fragments: 64 weight rows as four 16-row blocks (p), 32 activation
+  // rows as two (q), twice (j); k step ks is LDS chunks 4 ks .. 4 ks + 3 (lane
+  // l / 16). Byte offset of k step ks in a row block of a piece: one register
+  // per k step, everything else of the address is scalar or immediate
+  // (opaque, so that no other form of it takes registers through the loop).
   int foff[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     foff[ks] = (lane & 15) * kRB + (((4 * ks + (lane >> 4)) ^ tile_swz(lane & 15)) << 4);
     asm volatile("" : "+v"(foff[ks]));
   }
-  // fx[0]: X0, fx[1]: X1, fx[2]: the next stage's X0 where it is read ahead
-  V fw[2][4], fx[3][2][2];
-  auto read_w = [&](auto qc, int buf) LL_INLINE {
-    const int sb = buf * G::kStageB + decltype(qc)::value * kPieceB + wn * 64 * kRB;
+  V fw[2][4], fx[3][2][2];  // [ks][p]; [set][ks][q]
+  auto read_w = [&](int ks, int buf, int piece, int row) LL_INLINE {
+    const int sb = buf * G::kStageB + piece * kPieceB + row * kRB;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int p = 0; p < 4; ++p) fw[ks][p] = *(const V*)(smem + (sb + foff[ks]) + 16 * p * kRB);
+    for (int p = 0; p < 4; ++p) fw[ks][p] = *(const V*)(smem + (sb + foff[ks]) + 16 * p * kRB);
   };
-  auto read_x = [&](auto qc, int buf, V (&f)[2][2]) LL_INLINE {
-    const int sb = buf * G::kStageB + decltype(qc)::value * kPieceB + wm * 32 * kRB;
+  auto read_x = [&](int ks, int buf, int piece, int row, V (&f)[2][2]) LL_INLINE {
+    const int sb = buf * G::kStageB + piece * kPieceB + row * kRB;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int q = 0; q < 2; ++q) f[ks][q] = *(const V*)(smem + (sb + foff[ks]) + 16 * q * kRB);
+    for (int q = 0; q < 2; ++q) f[ks][q] = *(const V*)(smem + (sb + foff[ks]) + 16 * q * kRB);
   };
-  // the pieces of phase ph of the stage in buffer buf
-  auto read_phase = [&](auto phc, int buf) LL_INLINE {
-    constexpr int ph = decltype(phc)::value;
-    if constexpr (G::kAhead && ph == 0) {
+  // products i0 .. i1 - 1 of the 16 of k step ks: weight block h against both
+  // activation sets
+  auto multiply = [&](int h, int ks, int i0, int i1) LL_INLINE {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) fx[0][i / 2][i % 2] = fx[2][i / 2][i % 2];
+    for (int i = i0; i < i1; ++i) {
+      const int j = i / 8, p = i / 2 % 4, q = i % 2;
+      acc[h][j][p][q] = tile_mma(fw[ks][p], fx[j][ks][q], acc[h][j][p][q]);
     }
-    read_w(std::integral_constant<int, G::first(ph)>{}, buf);
-    if constexpr (G::kAhead) {
-      if constexpr (ph == 0) read_x(std::integral_constant<int, 1>{}, buf, fx[1]);
-      else read_x(std::integral_constant<int, 3>{}, 1 - buf, fx[2]);
-    } else if constexpr (ph == 0) {
-      read_x(std::integral_constant<int, 1>{}, buf, fx[0]);
-    }
-  };
-  // products of phase ph; full: both k steps (a half stage has one)
-  auto multiply = [&](auto phc, bool full) LL_INLINE {
-    constexpr int h = decltype(phc)::value;
-    auto step = [&](int ks) LL_INLINE {
-#pragma unroll
-      for (int j = 0; j < NXP; ++j)
-#pragma unroll
-        for (int p = 0; p < 4; ++p)
-#pragma unroll
-          for (int q = 0; q < 2; ++q)
-            acc[h][j][p][q] = tile_mma(fw[ks][p], fx[j][ks][q], acc[h][j][p][q]);
-    };
-    step(0);
-    if (full) step(1);
   };
 
-  // ---- epilogue. acc[h][j][p][q][i] = C[m][n] with m = m0 + 128 j + 32 wm
-  // + 16 q + l % 16 and n = n0 + (the 64 columns of h and wn) + 16 p +
-  // 4 (l / 16) + i. A lane's run of 4 columns is 8 or 16 bytes, so the rows
+  // ---- epilogue. acc[h][j][p][q][i] = C[m][n] with m = m0 + (the 32 rows of
+  // j and wm) + 16 q + l % 16 and n = n0 + (the 64 columns of h and wn) +
+  // 16 p + 4 (l / 16) + i. A lane's run of 4 columns is 8 or 16 bytes, so the rows
   // are turned through the wave's own piece of LDS: stores of whole 128-byte
   // (64-byte where the piece is smaller) row segments, 16 bytes per lane.
-  constexpr int kCB = G::kEpB >= 4096 && !(kSilu && NWP == 1) ? 128 : 64;  // bytes per row segment
+  constexpr int kCB = G::kEpB >= 4096 && !(kSilu && !kPP) ? 128 : 64;  // bytes per row segment
   constexpr int kRowsPI = 1024 / kCB;                 // rows per store instruction
   constexpr int kSegCols = kCB / (int)sizeof(TO);     // columns per segment
-  constexpr int kOutB = NWP * NXP * 64 * 32 * (int)sizeof(TO) / (kSilu ? 2 : 1);  // bytes per wave
+  constexpr int kOutB = NH * 2 * 64 * 32 * (int)sizeof(TO) / (kSilu ? 2 : 1);  // bytes per wave
   constexpr int kStores = kOutB / 1024;
   char* const ep = smem + kNst * G::kStageB + wave * G::kEpB;
   auto ep_swz = [](int row) LL_INLINE { return kCB == 128 ? (row & 7) : ((row >> 1) & 3); };
@@ -435,7 +408,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
     tile_coords<G>(a, item - sp * tiles, m0, n0);
     const __amdgpu_buffer_rsrc_t yres = __builtin_amdgcn_make_buffer_rsrc(
         (char*)a.Y + (int64_t)sp * a.split_b, (short)0, a.y_bytes, 0x00020000);
-    const int mw = m0 + wm * 32;
+    const int mw = m0 + wm * (kPP ? 32 : 64);
+    constexpr int kMj = kPP ? 128 : 32;  // rows between the two activation sets
     // the lane as a value of its own: nothing that follows from it is
     // computed ahead of the main loop and held in registers through it
     int el = lane;
@@ -444,21 +418,21 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
     // The per-row and per-column factors are loaded before the first store
     // that needs them, so the wave waits for them (and for the copies in
     // flight ahead of them) once, not once per store.
-    float st[NXP][2];
+    float st[2][2];
 #pragma unroll
-    for (int j = 0; j < NXP; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         st[j][q] = 1.f;
         if constexpr (EPI == EPI_DEQ || EPI == EPI_DEQ_SILU)
-          st[j][q] = a.s_tok[min(mw + 128 * j + 16 * q + lr, a.M - 1)];
+          st[j][q] = a.s_tok[min(mw + kMj * j + 16 * q + lr, a.M - 1)];
       }
     if constexpr (!kSilu) {
       typedef TO V4 __attribute__((ext_vector_type(4)));
       const bool has_bias = EPI != EPI_I32 && EPI != EPI_PART && a.bias != nullptr;
 #pragma unroll
-      for (int h = 0; h < NWP; ++h) {
-        const int nh = n0 + (NWP == 2 ? (2 * wn + h) * 64 : wn * 64);
+      for (int h = 0; h < NH; ++h) {
+        const int nh = n0 + (kPP ? 2 * wn + h : wn) * 64;
         int nl[4];  // in-range column groups for the loads
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -473,9 +447,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
         float sc[4][4];
         if constexpr (EPI == EPI_DEQ) tile_scales<4>(a.s_ch, a.s_ch_dtype, nl, sc);
 #pragma unroll
-        for (int j = 0; j < NXP; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
           for (int p = 0; p < 4; ++p) {
+            __builtin_amdgcn_sched_barrier(0);  // one group at a time (registers)
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
               TO o[4];
@@ -497,14 +472,14 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
               ep_put(16 * q + lr, 16 * p % kSegCols + 4 * lc, o);
             }
             if (16 * (p + 1) % kSegCols == 0)
-              ep_store(el, yres, mw + 128 * j, nh + 16 * (p + 1) - kSegCols, a.N);
+              ep_store(el, yres, mw + kMj * j, nh + 16 * (p + 1) - kSegCols, a.N);
           }
       }
     } else {
       // gate/up interleaved in 64-row blocks; this wave's channels:
-      //   2 x *: n0 / 2 + 64 wn + 16 p, gate acc[0][j][p], up acc[1][j][p]
-      //   1 x *: n0 / 2 + 32 wn + 16 p, gate acc[0][j][p], up acc[0][j][p + 2]
-      constexpr int NB = 2 * NWP;  // 16-channel blocks of this wave
+      //   256 x 256:  n0 / 2 + 64 wn + 16 p, gate acc[0][j][p], up acc[1][j][p]
+      //   the others: n0 / 2 + 32 wn + 16 p, gate acc[0][j][p], up acc[0][j][p + 2]
+      constexpr int NB = 2 * NH;  // 16-channel blocks of this wave
       const int I = a.N / 2;
       const int cw = n0 / 2 + wn * 16 * NB;
       float sc[2 * NB][4];  // scales of the gate channels, then the up channels
@@ -519,13 +494,14 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
         tile_scales<2 * NB>(a.s_ch, a.s_ch_dtype, cl, sc);
       }
 #pragma unroll
-      for (int j = 0; j < NXP; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int p = 0; p < NB; ++p) {
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int q = 0; q < 2; ++q) {
             const auto ga = acc[0][j][p][q];
-            const auto ua = NWP == 2 ? acc[NWP - 1][j][p][q] : acc[0][j][(p + 2) % 4][q];
+            const auto ua = kPP ? acc[NH - 1][j][p][q] : acc[0][j][(p + 2) % 4][q];
             TO o[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -545,46 +521,29 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
             ep_put(16 * q + lr, 16 * p % kSegCols + 4 * lc, o);
           }
           if (16 * (p + 1) % kSegCols == 0)
-            ep_store(el, yres, mw + 128 * j, cw + 16 * (p + 1) - kSegCols, I);
+            ep_store(el, yres, mw + kMj * j, cw + 16 * (p + 1) - kSegCols, I);
         }
     }
   };
 
-  // Ping-pong schedule. Waves 0-3 (group A) and 4-7 (group B) hold one wave
-  // of each SIMD (the dispatcher places wave w on SIMD w % 4). Time is cut
-  // into slots separated by workgroup barriers. In slot 2P group A reads the
-  // fragments of phase P and issues copies while group B multiplies phase
-  // P - 1; in slot 2P + 1 A multiplies phase P while B reads it. So each
-  // SIMD's matrix pipe has one wave with a run of MFMAs while the other
-  // wave's LDS reads and copies proceed. Ring invariants (R = kNst * kPh read
-  // phases in the ring):
-  //   * the pieces of read phase P have landed before slot 2P: each wave
-  //     issues them in its memory slot of phase P + 1 - R and waits for them
-  //     (vmcnt) before the barrier that ends slot 2P - 1, with the copies of
-  //     R - 2 later phases outstanding (wait_cnt);
-  //   * the buffer of read phase P - 1's pieces is refilled in the memory
-  //     slots of phase P (2P and 2P + 1), after the barrier that ends B's
-  //     read of them (slot 2P - 1, closed by lgkmcnt(0)).
-  // A wave writes a finished item's outputs in its first memory slot after
-  // the item's last stage, before that slot's copies, and does not wait for
-  // the stores: while the copies waited for were issued before the stores,
-  // the waits allow kStores more operations (a count at or below the exact
-  // one is always safe; vmcnt retires in issue order).
-  static_assert(G::wait_cnt(0) + kStores < 64 && G::wait_cnt(kPh - 1) + kStores < 64,
-                "vmcnt is a 6-bit counter");
-  constexpr int kAllow = kNst * kPh - 3;  // phases after an epilogue whose waits it may outlast
-  int since_ep = 64;                      // phases since this wave's last epilogue
-  auto wait_for = [&](auto qc) LL_INLINE {
-    constexpr int n = G::wait_cnt(decltype(qc)::value);
-    if (since_ep <= kAllow) tile_vm_wait<n + kStores>();
-    else tile_vm_wait<n>();
+  // Waits for the copies of the pieces read next. A finished item's stores are
+  // not waited for: while the copies waited for were issued before them
+  // (since_ep phases or stages after the epilogue, at most kAllow), the wait
+  // allows kStores more operations (a count at or below the exact one is
+  // always safe; vmcnt retires in issue order).
+  static_assert(G::kInFlight + kStores < 64, "vmcnt is a 6-bit counter");
+  constexpr int kAllow = kPP ? 1 : kNst - 2;
+  int since_ep = 64;
+  auto wait_next = [&]() LL_INLINE {
+    if (since_ep <= kAllow) tile_vm_wait<G::kInFlight + kStores>();
+    else tile_vm_wait<G::kInFlight>();
     ++since_ep;
   };
-  auto ph_const = [](auto f) LL_INLINE {  // calls f(integral_constant<0..kPh-1>) in order
-    f(std::integral_constant<int, 0>{});
-    if constexpr (kPh > 1) f(std::integral_constant<int, 1>{});
+  auto finish = [&](int item) LL_INLINE {
+    epilogue(item);
+    zero_acc();
+    since_ep = 0;
   };
-  const bool group_a = wave < 4;
   // cursor of the multiplications
   int cur_i = i_first, cur_k, cur_ke;
   auto cur_item = [&]() LL_INLINE {
@@ -593,54 +552,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
     cur_ke = min(cur_k + a.kps, a.nk);
   };
   cur_item();
-  constexpr std::integral_constant<int, 0> c0{};
-  constexpr std::integral_constant<int, kPh - 1> ph_last{};
-  // prologue: every read phase of the ring but the last one (after the first
-  // X0 where it is read ahead, which both groups read before the first slot)
-  if constexpr (G::kAhead) issue_piece(std::integral_constant<int, 3>{});
-#pragma unroll
-  for (int s = 0; s < kNst; ++s)
-    ph_const([&](auto ph) LL_INLINE {
-      if (s < kNst - 1 || decltype(ph)::value < kPh - 1) issue(ph);
-    });
-  tile_vm_wait<G::wait_cnt(0)>();
-  tile_barrier();
-  if constexpr (G::kAhead) {
-    read_x(std::integral_constant<int, 3>{}, 0, fx[2]);
-    tile_barrier();
-  }
   int buf = 0;
   bool more = true;
-  // sched_barrier keeps every instruction inside its slot (MFMAs touch no
-  // memory, so nothing else stops the scheduler moving them across barriers)
-  auto stage_a = [&]() LL_INLINE {
-    const bool full = !(a.half && cur_k == a.nk - 1);
-    const bool last = cur_k + 1 == cur_ke;  // the item's last stage
-    const int nbuf = buf == kNst - 1 ? 0 : buf + 1;
-    ph_const([&](auto phc) LL_INLINE {
-      constexpr int ph = decltype(phc)::value;
-      constexpr std::integral_constant<int, (ph + 1) % kPh> nxt{};
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_setprio(1);
-      multiply(phc, full);
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_sched_barrier(0);
-      wait_for(nxt);
-      tile_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (ph == kPh - 1) {
-        if (last) {
-          epilogue(cur_i);
-          zero_acc();
-          since_ep = 0;
-        }
-      }
-      read_phase(nxt, ph == kPh - 1 ? nbuf : buf);
-      issue(phc);
-      __builtin_amdgcn_sched_barrier(0);
-      tile_barrier();
-    });
-    buf = nbuf;
+  auto cur_next = [&](bool last) LL_INLINE {
+    buf = buf == kNst - 1 ? 0 : buf + 1;
     if (!last) {
       ++cur_k;
     } else {
@@ -649,54 +564,212 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tile_kernel(TileArgs a) {
       if (more) cur_item();
     }
   };
-  int done = -1;  // group B: item whose outputs are still in the accumulators
-  auto stage_b = [&]() LL_INLINE {
-    const bool full = !(a.half && cur_k == a.nk - 1);
-    const bool last = cur_k + 1 == cur_ke;
-    ph_const([&](auto phc) LL_INLINE {
+  // sched_barrier keeps every instruction inside its slot (MFMAs touch no
+  // memory, so nothing else stops the scheduler moving them across barriers)
+  if constexpr (kPP) {
+    // Ping-pong schedule. Waves 0-3 (group A) and 4-7 (group B) hold one wave
+    // of each SIMD (the dispatcher places wave w on SIMD w % 4). Time is cut
+    // into slots separated by workgroup barriers; phase P is P / 2's W0 or W1
+    // half. In slot 2P group A reads the fragments of phase P and issues
+    // copies while group B multiplies phase P - 1; in slot 2P + 1 A multiplies
+    // phase P while B reads it. So each SIMD's matrix pipe has one wave with a
+    // run of MFMAs while the other wave's LDS reads and copies proceed. Ring
+    // invariants (four phases in the ring):
+    //   * the pieces of phase P have landed before slot 2P: each wave issues
+    //     them in its memory slot of phase P - 3 and waits for them before the
+    //     barrier that ends slot 2P - 1, with two later phases outstanding;
+    //   * the buffers of phase P - 1's pieces are refilled in the memory slots
+    //     of phase P (2P and 2P + 1), after the barrier that ends B's read of
+    //     them (slot 2P - 1, closed by lgkmcnt(0)).
+    // A wave writes a finished item's outputs in its first memory slot after
+    // the item's last stage, before that slot's copies.
+    auto issue = [&](auto phc) LL_INLINE {
+      if constexpr (decltype(phc)::value == 0) {
+        issue_piece(c0);
+        issue_piece(c1);
+      } else {
+        issue_piece(c2);
+        issue_next();
+        issue_piece(c3);
+      }
+    };
+    auto read_x0 = [&](int b) LL_INLINE {
+      read_x(0, b, 3, wm * 32, fx[2]);
+      read_x(1, b, 3, wm * 32, fx[2]);
+    };
+    auto read_phase = [&](auto phc, int b) LL_INLINE {
       constexpr int ph = decltype(phc)::value;
-      constexpr std::integral_constant<int, (ph + 1) % kPh> nxt{};
-      constexpr std::integral_constant<int, (ph + kPh - 1) % kPh> prv{};
+      if constexpr (ph == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fx[0][i / 2][i % 2] = fx[2][i / 2][i % 2];
+      }
+      read_w(0, b, 2 * ph, wn * 64);
+      read_w(1, b, 2 * ph, wn * 64);
+      if constexpr (ph == 0) {
+        read_x(0, b, 1, wm * 32, fx[1]);
+        read_x(1, b, 1, wm * 32, fx[1]);
+      } else {
+        read_x0(1 - b);
+      }
+    };
+    auto multiply_phase = [&](auto phc, bool full) LL_INLINE {  // a half stage has one k step
+      __builtin_amdgcn_s_setprio(1);
+      multiply(decltype(phc)::value, 0, 0, 16);
+      if (full) multiply(decltype(phc)::value, 1, 0, 16);
+      __builtin_amdgcn_s_setprio(0);
+    };
+    // prologue: every phase of the ring but the last one, after the first X0,
+    // which both groups read before the first slot
+    issue_piece(c3);
+    issue(c0);
+    issue(c1);
+    issue(c0);
+    tile_vm_wait<G::kInFlight>();
+    tile_barrier();
+    read_x0(0);
+    tile_barrier();
+    auto phase_a = [&](auto phc, bool full, bool last) LL_INLINE {
+      constexpr int ph = decltype(phc)::value;
+      constexpr std::integral_constant<int, 1 - ph> nxt{};
+      __builtin_amdgcn_sched_barrier(0);
+      multiply_phase(phc, full);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_next();
+      tile_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (ph == 1) {
+        if (last) finish(cur_i);
+      }
+      read_phase(nxt, ph == 1 ? 1 - buf : buf);
+      issue(phc);
+      __builtin_amdgcn_sched_barrier(0);
+      tile_barrier();
+    };
+    int done = -1;  // group B: item whose outputs are still in the accumulators
+    auto phase_b = [&](auto phc, bool full) LL_INLINE {
+      constexpr int ph = decltype(phc)::value;
+      constexpr std::integral_constant<int, 1 - ph> prv{};
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (ph == 0) {
         if (done >= 0) {
-          epilogue(done);
-          zero_acc();
-          since_ep = 0;
+          finish(done);
           done = -1;
         }
       }
       read_phase(phc, buf);
       issue(prv);
       __builtin_amdgcn_sched_barrier(0);
-      wait_for(nxt);
+      wait_next();
       tile_barrier();
       __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_setprio(1);
-      multiply(phc, full);
-      __builtin_amdgcn_s_setprio(0);
+      multiply_phase(phc, full);
       __builtin_amdgcn_sched_barrier(0);
       tile_barrier();
-    });
-    buf = buf == kNst - 1 ? 0 : buf + 1;
-    if (!last) {
-      ++cur_k;
+    };
+    if (wave < 4) {
+      read_phase(c0, 0);
+      issue(c1);
+      tile_barrier();
+      while (more) {
+        const bool full = !(a.half && cur_k == a.nk - 1);
+        const bool last = cur_k + 1 == cur_ke;  // the item's last stage
+        phase_a(c0, full, last);
+        phase_a(c1, full, last);
+        cur_next(last);
+      }
     } else {
-      done = cur_i;
-      cur_i += g8;
-      more = cur_i < i_end;
-      if (more) cur_item();
+      tile_barrier();
+      while (more) {
+        const bool full = !(a.half && cur_k == a.nk - 1);
+        const bool last = cur_k + 1 == cur_ke;
+        phase_b(c0, full);
+        phase_b(c1, full);
+        if (last) done = cur_i;
+        cur_next(last);
+      }
+      epilogue(done);
     }
-  };
-  if (group_a) {
-    read_phase(c0, 0);
-    issue(ph_last);
-    tile_barrier();
-    while (more) stage_a();
   } else {
+    // Every wave alike, one barrier per stage. At the top of stage t its
+    // fragments are in registers (set t % 2); the barrier says that stage t + 1
+    // has landed and that everybody has read stage t, whose buffer takes stage
+    // t + kNst. The 16 fragment reads of stage t + 1 into the other set and
+    // those copies go out between the 32 MFMAs of stage t, so neither LDS
+    // latency nor the copies' issue holds them up. (The reads follow the first
+    // MFMA: the compiler waits for every outstanding LDS read where it first
+    // uses one.)
+    V gw[2][2][4], gx[2][2][2][2];  // [set][ks][p]; [set][ks][j][q]
+    const int wrow = (wn & 1) * 64, wpc = NWP == 2 ? (wn >> 1) * 2 : 0;
+    auto read_frag = [&](auto setc, int b, int r) LL_INLINE {
+      constexpr int set = decltype(setc)::value;
+      const int ks = r / 8, i = r % 8;
+      if (i < 4) {
+        const int sb = b * G::kStageB + wpc * kPieceB + wrow * kRB;
+        gw[set][ks][i] = *(const V*)(smem + (sb + foff[ks]) + 16 * i * kRB);
+      } else {
+        const int sb = b * G::kStageB + kPieceB + wm * 64 * kRB;
+        gx[set][ks][(i - 4) / 2][i % 2] = *(const V*)(smem + (sb + foff[ks]) + 16 * (i - 4) * kRB);
+      }
+    };
+    auto mul = [&](auto setc, int i) LL_INLINE {  // MFMA i of the stage's 32
+      constexpr int set = decltype(setc)::value;
+      const int ks = i / 16, j = i / 8 % 2, p = i / 2 % 4, q = i % 2;
+      acc[0][j][p][q] = tile_mma(gw[set][ks][p], gx[set][ks][j][q], acc[0][j][p][q]);
+    };
+    auto copy = [&](int i) LL_INLINE {  // copy i of the stage's kCopies
+      if constexpr (kDma == 4) {
+        if (i < 4) issue_copy(c0, i);
+        else issue_copy(c1, i - 4);
+      } else {
+        if (i < 2) issue_copy(c0, i);
+        else if (i < 4) issue_copy(c1, i - 2);
+        else issue_copy(c2, i - 4);
+      }
+    };
+    constexpr int kCopies = G::kPieces * kDma;
+    static_assert(kCopies <= 8, "a copy per four MFMAs");
+#pragma unroll
+    for (int t = 0; t < kNst; ++t) {
+#pragma unroll
+      for (int i = 0; i < kCopies; ++i) copy(i);
+      issue_next();
+    }
+    tile_vm_wait<(kNst - 1) * kCopies>();
     tile_barrier();
-    while (more) stage_b();
-    epilogue(done);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) read_frag(c0, 0, r);
+    auto stage = [&](auto setc) LL_INLINE {
+      constexpr int set = decltype(setc)::value;
+      constexpr std::integral_constant<int, 1 - set> other{};
+      const bool last = cur_k + 1 == cur_ke;
+      const int nbuf = buf == kNst - 1 ? 0 : buf + 1;
+      wait_next();
+      tile_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          mul(setc, 4 * g + i);
+          // int8: keeps the sum in one place (the compiler otherwise gives each
+          // product's result new registers and runs out of them)
+          if constexpr (sizeof(T) == 1) asm volatile("" : "+v"(acc[0][(4 * g + i) / 8 % 2][(4 * g + i) / 2 % 4][i % 2]));
+          __builtin_amdgcn_sched_barrier(0);
+          if (i % 2 == 0) read_frag(other, nbuf, 2 * g + i / 2);
+          if (i == 3 && g < kCopies) copy(g);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      issue_next();
+      if (last) finish(cur_i);
+      cur_next(last);
+    };
+    while (true) {
+      stage(c0);
+      if (!more) break;
+      stage(c1);
+      if (!more) break;
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   tile_vm_wait<0>();
@@ -738,21 +811,26 @@ struct TilePlan {
 // Tile geometry and k splits by a cost in us, fitted to a sweep of every
 // geometry and split count over M 96 .. 24000 at the 3B and 1.5B projections
 // (cold weights): a stage costs 1.15 us with few workgroups and 1.5 with all
-// CUs busy (256 x 256), 0.87 .. 1.0 (256 x 128), 0.55 (128 x 128); an item
-// 6, 2 and 3.7 us of fill and stores; the reduction of splits one more launch
+// CUs busy (256 x 256), 0.76 .. 0.93 (256 x 128), 0.50 (128 x 128); an item
+// 6, 2 and 3.3 us of fill and stores; the reduction of splits one more launch
 // and the partials' bytes both ways. So large outputs take 256 x 256 tiles
 // (M = 24,000, gate/up: 1736 us against 2244 and 2702), outputs of few tiles
 // smaller ones and splits (333 x 2048, K = 11008: 33 us with 128 x 128 tiles
 // in 5 splits, 98 unsplit, 197 as 16 tiles of 256 x 256), and what lies
 // between follows the rounds its tiles take (600 x 22016: 71 us in two
 // rounds of 256 x 128, 97 in two of 256 x 256).
-TilePlan plan_tiles(int64_t M, int64_t N, int64_t nk, int64_t max_splits, int cus) {
+// A K that ends in half a stage runs on the 256 x 256 form, the only one that
+// can leave out a k step; int8 has no 128 x 128 form (its sums and two
+// fragment sets do not fit the registers).
+TilePlan plan_tiles(int64_t M, int64_t N, int64_t K_b, int es, int64_t max_splits, int cus) {
+  const int64_t nk = ll_cdiv(K_b, kRB);
+  const int geos = K_b % kRB != 0 ? 1 : es == 1 ? 2 : 3;
   static const int tn[3] = {256, 256, 128}, tm[3] = {256, 128, 128};
-  static const double stage_us[3] = {1.15, 0.87, 0.55}, busy_us[3] = {0.35, 0.13, 0.0};
-  static const double item_us[3] = {6.0, 2.0, 3.7};
+  static const double stage_us[3] = {1.15, 0.76, 0.50}, busy_us[3] = {0.35, 0.17, 0.0};
+  static const double item_us[3] = {6.0, 2.0, 3.3};
   TilePlan best = {0, 1, (int)nk};
   double best_us = 1e30;
-  for (int g = 0; g < 3; ++g) {
+  for (int g = 0; g < geos; ++g) {
     const int64_t tiles = (int64_t)ll_cdiv(M, tm[g]) * ll_cdiv(N, tn[g]);
     for (int64_t sp = 1; sp <= max_splits; ++sp) {
       if (sp > 1 && (sp * kMinSplitStages > nk || tiles * sp > cus)) break;
@@ -804,7 +882,7 @@ int launch_geo(const TileArgs& a0, const TilePlan& plan, int cus, hipStream_t st
     a.group_m = tile_group_m(tiles_n, a.nk);
     const int64_t per = ((int64_t)a.tiles_m * a.tiles_n * a.splits + 7) / 8;
     const int64_t grid = 8 * std::min<int64_t>(per, std::max(1, cus / 8));
-    hipLaunchKernelGGL((gemm_tile_kernel<T, TO, EPI, G>), dim3((unsigned)grid), dim3(kThreads),
+    hipLaunchKernelGGL((gemm_tile_kernel<T, TO, EPI, G>), dim3((unsigned)grid), dim3(G::kThreads),
                        G::kLds, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -819,7 +897,9 @@ template <typename T, typename TO, int EPI>
 int launch_plan(const TileArgs& a, const TilePlan& plan, int cus, hipStream_t stream) {
   if (plan.geo == 0) return launch_geo<T, TO, EPI, TileGeo<2, 2>>(a, plan, cus, stream);
   if (plan.geo == 1) return launch_geo<T, TO, EPI, TileGeo<2, 1>>(a, plan, cus, stream);
-  return launch_geo<T, TO, EPI, TileGeo<1, 1>>(a, plan, cus, stream);
+  if constexpr (sizeof(T) == 2) return launch_geo<T, TO, EPI, TileGeo<1, 1>>(a, plan, cus, stream);
+  ll_set_error("gemm tiles: no 128 x 128 form for int8");
+  return LL_ERR_UNSUPPORTED;
 }
 
 // one k split, outputs in their final form
@@ -828,7 +908,7 @@ int launch_tiles(const TileArgs& a, hipStream_t stream) {
   int cus = 0;
   const int rc = ll_device_cus(&cus);
   if (rc != LL_OK) return rc;
-  return launch_plan<T, TO, EPI>(a, plan_tiles(a.M, a.N, a.nk, 1, cus), cus, stream);
+  return launch_plan<T, TO, EPI>(a, plan_tiles(a.M, a.N, a.K_b, sizeof(T), 1, cus), cus, stream);
 }
 
 // Sum of the k splits' partials [splits][M][N], in split order, finished as
@@ -879,7 +959,7 @@ int launch_tiles_ws(const TileArgs& a, void* ws, int64_t ws_bytes, hipStream_t s
   if (rc != LL_OK) return rc;
   const int64_t split_b = (int64_t)a.M * a.N * 4;
   const int64_t room = ws != nullptr && (uintptr_t)ws % 16 == 0 ? ws_bytes / split_b : 0;
-  const TilePlan plan = plan_tiles(a.M, a.N, a.nk, std::max<int64_t>(1, room), cus);
+  const TilePlan plan = plan_tiles(a.M, a.N, a.K_b, sizeof(T), std::max<int64_t>(1, room), cus);
   if (plan.splits == 1) return launch_plan<T, TO, EPI>(a, plan, cus, stream);
   TileArgs pa = a;
   pa.Y = ws;
@@ -922,6 +1002,7 @@ TileArgs make_args(const void* X, int64_t ldx_b, const void* W, int64_t ldw_b, i
   a.X = (const char*)X; a.ldx_b = ldx_b;
   a.W = (const char*)W; a.ldw_b = ldw_b;
   a.M = (int)M; a.N = (int)N;
+  a.K_b = (int)K_b;
   a.nk = a.kps = ll_cdiv(K_b, kRB);
   a.half = K_b % kRB != 0;
   a.Y = Y; a.ldy = ldy;
@@ -980,7 +1061,7 @@ extern "C" int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K,
   if (M <= 64 || N <= 0 || N % 4 != 0 || K <= 0 || (elem_bytes != 1 && elem_bytes != 2) ||
       (K * elem_bytes) % kKUnit != 0)
     return 0;
-  const TilePlan p = plan_tiles(M, N, ll_cdiv(K * elem_bytes, kRB), kPlanCus, kPlanCus);
+  const TilePlan p = plan_tiles(M, N, K * elem_bytes, (int)elem_bytes, kPlanCus, kPlanCus);
   return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
 }
 

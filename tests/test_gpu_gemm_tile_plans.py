@@ -24,6 +24,7 @@ def _excess(y, ref):
 @pytest.mark.parametrize("M,N,K,dtype,bias,split", [
     (65, 1536, 8960, torch.bfloat16, True, True),       # 128 x 128, many splits, last one shorter
     (128, 132, 4128, torch.float16, False, True),       # N % 8 == 4, half a stage at the end
+    (100, 260, 4096, torch.float16, True, True),        # N % 8 == 4, 128 x 128 in splits
     (129, 2048, 11008, torch.bfloat16, False, True),    # one row past a tile
     (600, 2048, 11008, torch.bfloat16, True, True),     # 256 x 128 in splits
     (1679, 1536, 8960, torch.float16, False, True),     # 256 x 256 in splits
@@ -62,16 +63,16 @@ def test_gemm_i8_splits_are_exact(cuda, M, N, K):
     assert torch.equal(_ops().gemm_i8_i32_tiled(xq.to(cuda), wq.to(cuda)).cpu(), acc)
 
 
-@pytest.mark.parametrize("M", [65, 129, 257, 700])
-def test_gate_up_silu_geometries_agree(cuda, M):
+@pytest.mark.parametrize("M,K", [(65, 64), (129, 192), (257, 160), (700, 320), (1100, 96)])
+def test_gate_up_silu_geometries_agree(cuda, M, K):
     """The fused epilogue of every geometry equals the product followed by
     silu_and_mul bit for bit (K sums run in the same order in all of them)."""
     g = torch.Generator().manual_seed(93)
-    I, K = 8960, 160  # half a stage at the end
+    I = 8960
     x = torch.randn(M, K, generator=g).half().to(cuda)
     w = (torch.randn(2 * I, K, generator=g) * 0.1).half().to(cuda)
     ops = _ops()
-    print(f"case: gate_up_silu geometry M={M}", flush=True)
+    print(f"case: gate_up_silu geometry M={M} K={K}", flush=True)
     want = ops.silu_and_mul(ops.gemm_tiled(x, w), out=torch.empty(M, I, dtype=x.dtype, device=cuda))
     assert torch.equal(ops.gate_up_silu_tiled(x, ops.interleave_gate_up(w)), want)
 
