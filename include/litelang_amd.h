@@ -595,6 +595,48 @@ int ll_probe_launch(void* dst, int64_t write_bytes, int64_t workgroups, hipStrea
 int ll_decode_attention_split_count(int64_t batch, int64_t kv_heads, int64_t head_dim,
                                     int64_t max_len_in_batch);
 
+/* ------------------------------------------------------------ record calls
+ * The same calls with their arguments in one record of 8-byte fields (pointers
+ * and flags widened to int64, floats to double, in the entry point's order):
+ * a caller whose foreign-function interface converts every argument by itself
+ * (Python's ctypes: 3 us for the 31 arguments of ll_decode_attention) packs
+ * the record in one step. They return what the entry point returns, or, where
+ * the workspace is smaller than the call wants, that size in bytes (> 0) with
+ * nothing launched; with `any_workspace` set, ll_call_gemm (M > 64) runs with
+ * the workspace it is given instead. */
+typedef struct {
+  int64_t x, x_row_stride, residual, residual_row_stride, gamma, out, out_row_stride, M, N;
+  double eps;
+  int64_t dtype, stream;
+} LLRmsnormCall;
+int64_t ll_call_rmsnorm(const LLRmsnormCall* c);
+
+typedef struct {
+  int64_t q, q_stride_b, q_stride_h, k_cache, k_stride_tok, k_stride_head, v_cache, v_stride_tok,
+      v_stride_head, req_to_tokens, req_to_tokens_stride, b_req_idx, req_idx_i64, b_seq_len,
+      seq_len_i64, out, out_stride_b, out_stride_h, batch, q_heads, kv_heads, head_dim,
+      max_len_in_batch;
+  double sm_scale;
+  int64_t dtype, workspace, workspace_bytes, stream;
+} LLDecodeAttentionCall;
+int64_t ll_call_decode_attention(const LLDecodeAttentionCall* c);
+
+typedef struct {
+  int64_t q, q_stride_tok, q_stride_h, k_cache, k_stride_tok, k_stride_head, v_cache, v_stride_tok,
+      v_stride_head, out, out_stride_tok, out_stride_h, req_to_tokens, req_to_tokens_stride,
+      b_req_idx, req_idx_i64, b_start_loc, start_loc_i64, b_seq_len, seq_len_i64, b_shared_seq_len,
+      shared_i64, batch, q_heads, kv_heads, head_dim, max_input_len;
+  double sm_scale;
+  int64_t dtype, stream;
+} LLPrefillAttentionCall;
+int64_t ll_call_prefill_attention(const LLPrefillAttentionCall* c);
+
+typedef struct {
+  int64_t X, ldx, W, ldw, bias, Y, ldy, M, N, K, dtype, workspace, workspace_bytes, any_workspace,
+      stream;
+} LLGemmCall;
+int64_t ll_call_gemm(const LLGemmCall* c);
+
 #ifdef __cplusplus
 }
 #endif

@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "liblitelang_amd.so")
@@ -17,6 +18,12 @@ P = ctypes.c_void_p
 I64 = ctypes.c_int64
 I32 = ctypes.c_int
 F32 = ctypes.c_float
+
+# packed records of the ll_call_* forms (LL*Call in include/litelang_amd.h)
+RMSNORM_CALL = struct.Struct("=9qd2q")
+DECODE_ATTENTION_CALL = struct.Struct("=23qd4q")
+PREFILL_ATTENTION_CALL = struct.Struct("=27qd2q")
+GEMM_CALL = struct.Struct("=15q")
 
 # name -> (restype, argtypes), mirroring include/litelang_amd.h
 SIGNATURES = {
@@ -115,6 +122,11 @@ SIGNATURES = {
                                  I64, I64, I64, I32, P, P]),
     "ll_decode_attention_split_count": (I32, [I64, I64, I64, I64]),
     "ll_probe_launch": (I32, [P, I64, I64, P]),
+    # record calls: the packed record (bytes)
+    "ll_call_rmsnorm": (I64, [ctypes.c_char_p]),
+    "ll_call_decode_attention": (I64, [ctypes.c_char_p]),
+    "ll_call_prefill_attention": (I64, [ctypes.c_char_p]),
+    "ll_call_gemm": (I64, [ctypes.c_char_p]),
 }
 
 

@@ -30,17 +30,21 @@ def token_decode_attention_flash_decoding(
     assert Lk in {16, 32, 64, 128}
     batch_size = q.size(0)
     calcu_shape1 = (batch_size, q_head_num, head_dim)
-    o_tensor = (
-        alloc_tensor_func(q.shape, dtype=q.dtype, device=q.device) if out is None else out
-    )
+    if out is not None:
+        o_tensor = out
+    elif alloc_tensor_func is torch.empty:
+        o_tensor = torch.empty_like(q, memory_format=torch.contiguous_format)
+    else:
+        o_tensor = alloc_tensor_func(q.shape, dtype=q.dtype, device=q.device)
+    same = q.shape == calcu_shape1
     ops.decode_attention(
-        q.view(calcu_shape1),
+        q if same else q.view(calcu_shape1),
         req_to_token_indexs,
         b_req_idx,
         b_seq_len,
         int(max_len_in_batch),
         cache_k,
         cache_v,
-        o_tensor.view(calcu_shape1),
+        o_tensor if same and o_tensor.shape == calcu_shape1 else o_tensor.view(calcu_shape1),
     )
     return o_tensor

@@ -31,14 +31,35 @@ def _idx(t: torch.Tensor, name: str) -> int:
         raise TypeError(f"{name}: index tensor must be int32 or int64, got {t.dtype}") from None
 
 
+_raw_stream = torch._C._cuda_getCurrentRawStream  # by device index, without a Stream object
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _dev(*ts: torch.Tensor) -> None:
     for t in ts:
         if t is not None and not t.is_cuda:
             raise ValueError("lite_lang_amd ops need device tensors (got a CPU tensor)")
+
+
+def _call(fn, rec, fields, name, ws_name, ws_at, t):
+    """A record call (ll_call_*) with the current stream's workspace `ws_name`
+    as it stands in the fields ws_at and ws_at + 1, again with a larger one
+    when the library asks for it."""
+    idx = t.get_device()
+    stream = _raw_stream(idx)
+    buf = _WS.get((idx, stream, ws_name))
+    if buf is not None:
+        fields[ws_at], fields[ws_at + 1] = buf.data_ptr(), buf.numel()
+    fields[-1] = stream
+    rc = fn(rec.pack(*fields))
+    if rc > 0:
+        return rc
+    if rc != 0:
+        _lib.check(rc, name)
+    return 0
 
 
 # ------------------------------------------------------------------ workspaces
@@ -60,7 +81,7 @@ _RETIRED: list[torch.Tensor] = []
 
 def _ws_key(device: torch.device, name: str):
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    return (idx, torch.cuda.current_stream(idx).cuda_stream, name)
+    return (idx, _raw_stream(idx), name)
 
 
 def workspace(device: torch.device, name: str, nbytes: int) -> torch.Tensor:
@@ -118,20 +139,18 @@ def decode_attention(q, req_to_tokens, b_req_idx, b_seq_len, max_len_in_batch, c
     assert req_to_tokens.stride(-1) == 1
     if sm_scale is None:
         sm_scale = 1.0 / (D ** 0.5)
-    max_len = int(max_len_in_batch)
-    nbytes = _L.ll_decode_attention_workspace_size(B, H, KVH, D, max_len)
-    ws = workspace(q.device, "decode_attention", nbytes)
-    rc = _L.ll_decode_attention(
-        q.data_ptr(), q.stride(0), q.stride(1),
-        cache_k.data_ptr(), cache_k.stride(0), cache_k.stride(1),
-        cache_v.data_ptr(), cache_v.stride(0), cache_v.stride(1),
-        req_to_tokens.data_ptr(), req_to_tokens.stride(0),
-        b_req_idx.data_ptr(), _idx(b_req_idx, "b_req_idx"),
-        b_seq_len.data_ptr(), _idx(b_seq_len, "b_seq_len"),
-        out.data_ptr(), out.stride(0), out.stride(1),
-        B, H, KVH, D, max_len, float(sm_scale), dtype_code(q),
-        ws.data_ptr(), ws.numel(), _stream(q))
-    _lib.check(rc, "ll_decode_attention")
+    qs, ks, vs, os_ = q.stride(), cache_k.stride(), cache_v.stride(), out.stride()
+    fields = [q.data_ptr(), qs[0], qs[1], cache_k.data_ptr(), ks[0], ks[1], cache_v.data_ptr(),
+              vs[0], vs[1], req_to_tokens.data_ptr(), req_to_tokens.stride(0),
+              b_req_idx.data_ptr(), _idx(b_req_idx, "b_req_idx"),
+              b_seq_len.data_ptr(), _idx(b_seq_len, "b_seq_len"), out.data_ptr(), os_[0], os_[1],
+              B, H, KVH, D, int(max_len_in_batch), float(sm_scale), dtype_code(q), 0, 0, 0]
+    need = _call(_L.ll_call_decode_attention, _lib.DECODE_ATTENTION_CALL, fields,
+                 "ll_decode_attention", "decode_attention", 25, q)
+    if need:
+        workspace(q.device, "decode_attention", need)
+        _call(_L.ll_call_decode_attention, _lib.DECODE_ATTENTION_CALL, fields,
+              "ll_decode_attention", "decode_attention", 25, q)
     return out
 
 
@@ -188,17 +207,14 @@ def prefill_attention(q, k, v, o, b_req_idx, b_start_loc, b_seq_len, max_input_l
     if b_shared_seq_len is not None:
         _dev(b_shared_seq_len)
         sh_ptr, sh64 = b_shared_seq_len.data_ptr(), _idx(b_shared_seq_len, "b_shared_seq_len")
-    rc = _L.ll_prefill_attention(
-        q.data_ptr(), q.stride(0), q.stride(1),
-        k.data_ptr(), k.stride(0), k.stride(1),
-        v.data_ptr(), v.stride(0), v.stride(1),
-        o.data_ptr(), o.stride(0), o.stride(1),
-        req_to_tokens.data_ptr(), req_to_tokens.stride(0),
+    qs, ks, vs, os_ = q.stride(), k.stride(), v.stride(), o.stride()
+    rc = _L.ll_call_prefill_attention(_lib.PREFILL_ATTENTION_CALL.pack(
+        q.data_ptr(), qs[0], qs[1], k.data_ptr(), ks[0], ks[1], v.data_ptr(), vs[0], vs[1],
+        o.data_ptr(), os_[0], os_[1], req_to_tokens.data_ptr(), req_to_tokens.stride(0),
         b_req_idx.data_ptr(), _idx(b_req_idx, "b_req_idx"),
         b_start_loc.data_ptr(), _idx(b_start_loc, "b_start_loc"),
-        b_seq_len.data_ptr(), _idx(b_seq_len, "b_seq_len"),
-        sh_ptr or None, sh64,
-        B, H, KVH, D, int(max_input_len), float(sm_scale), dtype_code(q), _stream(q))
+        b_seq_len.data_ptr(), _idx(b_seq_len, "b_seq_len"), sh_ptr, sh64,
+        B, H, KVH, D, int(max_input_len), float(sm_scale), dtype_code(q), _stream(q)))
     _lib.check(rc, "ll_prefill_attention")
     return o
 
@@ -208,17 +224,20 @@ def rmsnorm(x, gamma, eps, residual=None, out=None):
     """out = rmsnorm(x [+ residual]) * gamma; with residual, x is updated in place."""
     _dev(x, gamma, residual, out)
     assert x.ndim == 2 and x.shape[1] == gamma.shape[0]
-    assert x.stride(1) == 1 and gamma.stride(0) == 1
+    xs = x.stride()
+    assert xs[1] == 1 and gamma.stride(0) == 1
     if out is None:
         out = torch.empty_like(x)
-    assert out.shape == x.shape and out.stride(1) == 1
-    r_ptr, r_rs = (None, 0)
+    os_ = out.stride()
+    assert out.shape == x.shape and os_[1] == 1
+    r_ptr, r_rs = 0, 0
     if residual is not None:
         assert residual.shape == x.shape and residual.stride(1) == 1
         r_ptr, r_rs = residual.data_ptr(), residual.stride(0)
-    rc = _L.ll_rmsnorm(x.data_ptr(), x.stride(0), r_ptr, r_rs, gamma.data_ptr(), out.data_ptr(),
-                       out.stride(0), x.shape[0], x.shape[1], float(eps), dtype_code(x),
-                       _stream(x))
+    M, N = x.shape
+    rc = _L.ll_call_rmsnorm(_lib.RMSNORM_CALL.pack(
+        x.data_ptr(), xs[0], r_ptr, r_rs, gamma.data_ptr(), out.data_ptr(), os_[0], M, N,
+        float(eps), dtype_code(x), _stream(x)))
     _lib.check(rc, "ll_rmsnorm")
     return out
 
@@ -353,20 +372,16 @@ def gemm(x, w, bias=None, out=None):
     if out is None:
         out = torch.empty((M, N), dtype=x.dtype, device=x.device)
     assert out.shape == (M, N) and out.stride(1) == 1
-    ws_ptr, ws_n = (None, 0)
-    if M > 64:
-        if x.dtype != torch.float32:
-            ws_ptr, ws_n = optional_workspace(x.device, "gemm",
-                                              _L.ll_gemm_tiles_workspace_size(M, N, K, 2))
-    else:
-        nbytes = _L.ll_gemm_workspace_size(M, N, K)
-        if nbytes > 0:
-            ws = workspace(x.device, "gemm", nbytes)
-            ws_ptr, ws_n = ws.data_ptr(), ws.numel()
-    rc = _L.ll_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
-                    bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
-                    M, N, K, dtype_code(x), ws_ptr, ws_n, _stream(x))
-    _lib.check(rc, "ll_gemm")
+    fields = [x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
+              bias.data_ptr() if bias is not None else 0, out.data_ptr(), out.stride(0), M, N, K,
+              dtype_code(x), 0, 0, 0, 0]
+    need = _call(_L.ll_call_gemm, _lib.GEMM_CALL, fields, "ll_gemm", "gemm", 11, x)
+    if need:
+        if M > 64 and torch.cuda.is_current_stream_capturing():
+            fields[13] = 1  # nothing is allocated inside a capture: run with what there is
+        else:
+            workspace(x.device, "gemm", need)
+        _call(_L.ll_call_gemm, _lib.GEMM_CALL, fields, "ll_gemm", "gemm", 11, x)
     return out
 
 

@@ -75,3 +75,39 @@ def test_host_only_settings():
     rc = lib.ll_embedding_rmsnorm_epoch(256, 8, 8, 256, 0, 256, 8, 256, 256, 8, 4, 8,
                                         _lib.F32(1e-6), 2, 256, 256, 8, None, 256, 256, None)
     assert rc == -1 and b"slot-table" in lib.ll_last_error()
+
+
+def test_record_calls_match_their_entry_points():
+    """The packed records hold as many fields as the header declares, an empty
+    decode batch is accepted, a small workspace is answered with the size
+    wanted before anything is launched, and argument errors come through."""
+    import re
+    lib = _lib.load()
+    text = open(_lib.HEADER_PATH).read()
+    for name, rec in (("LLRmsnormCall", _lib.RMSNORM_CALL),
+                      ("LLDecodeAttentionCall", _lib.DECODE_ATTENTION_CALL),
+                      ("LLPrefillAttentionCall", _lib.PREFILL_ATTENTION_CALL),
+                      ("LLGemmCall", _lib.GEMM_CALL)):
+        body = re.search(r"typedef struct \{([^}]*)\} %s;" % name, text).group(1)
+        assert rec.size == 8 * len(re.findall(r"\w+(?=[,;])", body))
+    p = 4096  # never dereferenced
+    att = [p, 1, 1, p, 1, 1, p, 1, 1, p, 1, p, 0, p, 0, p, 1, 1, 40, 12, 2, 128, 600, 0.1, 2, p,
+           1024, 0]
+    pack = _lib.DECODE_ATTENTION_CALL.pack
+    assert lib.ll_call_decode_attention(pack(*att)) == \
+        lib.ll_decode_attention_workspace_size(40, 12, 2, 128, 600)
+    att[18] = 0
+    assert lib.ll_call_decode_attention(pack(*att)) == 0
+    att[0] = 0
+    assert lib.ll_call_decode_attention(pack(*att)) == -1
+    assert b"null pointer" in lib.ll_last_error()
+    gemm = [p, 2048, p, 2048, 0, p, 2048, 40, 2048, 2048, 2, 0, 0, 0, 0]
+    assert lib.ll_call_gemm(_lib.GEMM_CALL.pack(*gemm)) == lib.ll_gemm_workspace_size(40, 2048, 2048)
+    gemm[7] = 96
+    want = lib.ll_gemm_tiles_workspace_size(96, 2048, 2048, 2)
+    assert want > 0 and lib.ll_call_gemm(_lib.GEMM_CALL.pack(*gemm)) == want
+    gemm[0], gemm[13] = 0, 1
+    assert lib.ll_call_gemm(_lib.GEMM_CALL.pack(*gemm)) == -1
+    rms = [0, 8, 0, 0, p, p, 8, 4, 8, 1e-6, 2, 0]
+    assert lib.ll_call_rmsnorm(_lib.RMSNORM_CALL.pack(*rms)) == -1
+    assert b"null pointer" in lib.ll_last_error()
