@@ -257,6 +257,15 @@ int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t ldw, const 
  * int8); 0 where they do not split. With less they run one split. */
 int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K, int64_t elem_bytes);
 
+/* fp32 partial sums [splits][M][N] of the tile GEMM's product (bf16/fp16, the
+ * layout rules of ll_gemm_tiled), for the split-K consumers (ll_add_rmsnorm_splitk,
+ * ll_rope_kv_scatter_splitk, ll_decode_attention_rope_splitk). The split count
+ * is ll_gemm_tiles_splitk_count(M, N, K, dtype), 0 for shapes without a form. */
+int ll_gemm_tiles_splitk_count(int64_t M, int64_t N, int64_t K, int dtype);
+int ll_gemm_tiles_splitk(const void* X, int64_t ldx, const void* W, int64_t ldw, int64_t M,
+                         int64_t N, int64_t K, int dtype, float* part, int64_t part_bytes,
+                         hipStream_t stream);
+
 /* Copy of a [gate; up] weight ([2I, K], I % 128 == 0, elem_bytes 2 or 1)
  * with its rows interleaved in 64-row blocks (gate c..c+63, up c..c+63,
  * ...), the layout ll_gemm_gate_up_silu_tiled and

@@ -538,6 +538,26 @@ def gemm_splitk(x, w, part):
     return s
 
 
+def gemm_tiles_splitk_count(M, N, K, dtype) -> int:
+    """k splits of gemm_tiles_splitk's partials; 0 for shapes it does not cover."""
+    code = _DTYPES.get(dtype)
+    return 0 if code is None else int(_L.ll_gemm_tiles_splitk_count(M, N, K, code))
+
+
+def gemm_tiles_splitk(x, w, part):
+    """gemm_splitk on the tile GEMM (more than 64 rows): fp32 partials into
+    part, split count returned."""
+    _dev(x, w, part)
+    M, K = x.shape
+    N = w.shape[0]
+    assert w.shape[1] == K and x.stride(1) == 1 and w.stride(1) == 1 and x.dtype == w.dtype
+    assert part.dtype == torch.float32
+    rc = _L.ll_gemm_tiles_splitk(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), M, N, K,
+                                 dtype_code(x), part.data_ptr(), part.numel() * 4, _stream(x))
+    _lib.check(rc, "ll_gemm_tiles_splitk")
+    return gemm_tiles_splitk_count(M, N, K, x.dtype)
+
+
 class PackedWeight:
     """A [N, K] nn.Linear weight in the weight-streaming kernel's packed layout
     (ll_gemm_pack); keeps the logical shape next to the packed bytes."""
