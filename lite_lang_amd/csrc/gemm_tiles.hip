@@ -72,7 +72,16 @@ constexpr int kPieceB = 128 * kRB;  // a piece: 128 rows of one operand (16 KB)
 // stage, bounded by LDS (reads and copies of 96 KB per 128 x 128 stage): 0.74
 // and 0.49 us (few workgroups), against 0.87 and 0.56 with two groups taking
 // turns on 64 x 32 per wave (128 KB, and a barrier after each turn).
-template <int NWP_, int NXP_> struct TileGeo {
+//
+// NT: the weight copies are non-temporal, for one row tile (M <= 128) in one k
+// split, where every weight byte is read once and would only push the
+// activations out of L2 (96 rows, cold weights): gate/up + SiLU 26.9 -> 25.4
+// us (22016 x 2048) and 21.0 -> 20.2 (17920 x 1536), lm_head 157 -> 152 and
+// 110 -> 102. With two row tiles, which share the weights through L2, it
+// costs (160 rows, 151936 x 2048: 174 -> 204), and k splits lose too (2048 x
+// 11008: 19.0 -> 21.2; 1536 x 8960: 15.7 -> 18.2).
+template <int NWP_, int NXP_, bool NT_ = false> struct TileGeo {
+  static constexpr bool kNt = NT_;
   static constexpr int NWP = NWP_, NXP = NXP_;
   static constexpr int TN = 128 * NWP, TM = 128 * NXP;
   static constexpr int kPieces = NWP + NXP;
@@ -117,6 +126,11 @@ __device__ __forceinline__ i32x4 tile_mma(i32x4 a, i32x4 b, i32x4 c) {
 // the templates (a dependent call of this builtin drops the host launch stub).
 __device__ __forceinline__ void tile_dma16(const void* g, void* lds) {
   __builtin_amdgcn_global_load_lds(g, lds, 16, 0, 0);
+}
+
+// the same, non-temporal
+__device__ __forceinline__ void tile_dma16_nt(const void* g, void* lds) {
+  __builtin_amdgcn_global_load_lds(g, lds, 16, 0, 2 /* nt */);
 }
 
 template <int N_> __device__ __forceinline__ void tile_vm_wait() {
@@ -294,8 +308,10 @@ __global__ __launch_bounds__(G::kThreads, 2) void gemm_tile_kernel(TileArgs a) {
     const int64_t kb = past ? 0 : (int64_t)iss_k * kRB;
     uint32_t o = (soff[q][u] - tadj) & pmask;
     asm volatile("" : "+v"(o));  // no 64-bit form of it is held through the loop
-    tile_dma16((G::is_w(q) ? a.W : a.X) + kb + o,
-               smem + iss_buf * G::kStageB + q * kPieceB + (kWaves * u + wave) * 1024);
+    const char* src = (G::is_w(q) ? a.W : a.X) + kb + o;
+    char* dst = smem + iss_buf * G::kStageB + q * kPieceB + (kWaves * u + wave) * 1024;
+    if constexpr (G::kNt && G::is_w(q)) tile_dma16_nt(src, dst);
+    else tile_dma16(src, dst);
   };
   auto issue_piece = [&](auto qc) LL_INLINE {
 #pragma unroll
@@ -896,8 +912,13 @@ int launch_geo(const TileArgs& a0, const TilePlan& plan, int cus, hipStream_t st
 template <typename T, typename TO, int EPI>
 int launch_plan(const TileArgs& a, const TilePlan& plan, int cus, hipStream_t stream) {
   if (plan.geo == 0) return launch_geo<T, TO, EPI, TileGeo<2, 2>>(a, plan, cus, stream);
-  if (plan.geo == 1) return launch_geo<T, TO, EPI, TileGeo<2, 1>>(a, plan, cus, stream);
-  if constexpr (sizeof(T) == 2) return launch_geo<T, TO, EPI, TileGeo<1, 1>>(a, plan, cus, stream);
+  const bool nt = a.M <= 128 && plan.splits == 1;  // TileGeo: the weights are read once
+  if (plan.geo == 1)
+    return nt ? launch_geo<T, TO, EPI, TileGeo<2, 1, true>>(a, plan, cus, stream)
+              : launch_geo<T, TO, EPI, TileGeo<2, 1>>(a, plan, cus, stream);
+  if constexpr (sizeof(T) == 2)
+    return nt ? launch_geo<T, TO, EPI, TileGeo<1, 1, true>>(a, plan, cus, stream)
+              : launch_geo<T, TO, EPI, TileGeo<1, 1>>(a, plan, cus, stream);
   ll_set_error("gemm tiles: no 128 x 128 form for int8");
   return LL_ERR_UNSUPPORTED;
 }
