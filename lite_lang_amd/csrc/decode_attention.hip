@@ -905,33 +905,38 @@ __global__ __launch_bounds__(kCombWaves * 64) void decode_attn_combine_kernel(De
   for (int q = 0; q < DPL; ++q) op[lane + 64 * q] = ll_from_f32<T>(o[q]);
 }
 
-// Combine of one sequence per workgroup (HPW heads per wave, H <= 16 * HPW),
-// then the o_proj input quantisation of the stored row out[b] (H * D values):
-// codes by ll_quant_per_token's rule, or by *a.qstatic when set.
+// Combine of one sequence per workgroup, then the o_proj input quantisation of
+// the stored row out[b] (H * D values): codes by ll_quant_per_token's rule, or
+// by *a.qstatic when set. HPW > 0: a wave keeps its (at most HPW) heads in
+// registers between the two (H <= 16 * HPW); 0: any H, the second pass reads
+// the stored values back, each lane its own.
 template <typename T, int D, int HPW>
 __global__ __launch_bounds__(1024) void decode_attn_combine_quant_kernel(DecodeArgs a) {
   constexpr int DPL = D / 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int nw = blockDim.x >> 6;
   const int b = blockIdx.x;
-  float y[HPW][DPL];
   float amax = 0.f;
+  auto out_of = [&](int h) { return (T*)a.out + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + lane; };
+  auto merge = [&](int h, float (&y)[DPL]) {
+    float o[DPL];
+    combine_bh<D>(a, b * a.H + h, lane, o);
+    clear_bh<D>(a, b * a.H + h, lane);
 #pragma unroll
-  for (int k = 0; k < HPW; ++k) {
-    const int h = wave + k * nw;
-    if (h < a.H) {
-      float o[DPL];
-      combine_bh<D>(a, b * a.H + h, lane, o);
-      clear_bh<D>(a, b * a.H + h, lane);
-      T* op = (T*)a.out + (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
-#pragma unroll
-      for (int q = 0; q < DPL; ++q) {
-        const T v = ll_from_f32<T>(o[q]);
-        op[lane + 64 * q] = v;
-        y[k][q] = ll_to_f32(v);
-        amax = fmaxf(amax, fabsf(y[k][q]));
-      }
+    for (int q = 0; q < DPL; ++q) {
+      const T v = ll_from_f32<T>(o[q]);
+      out_of(h)[64 * q] = v;
+      y[q] = ll_to_f32(v);
+      amax = fmaxf(amax, fabsf(y[q]));
     }
+  };
+  float y[HPW > 0 ? HPW : 1][DPL];
+  if constexpr (HPW > 0) {
+#pragma unroll
+    for (int k = 0; k < HPW; ++k)
+      if (wave + k * nw < a.H) merge(wave + k * nw, y[k]);
+  } else {
+    for (int h = wave; h < a.H; h += nw) merge(h, y[0]);
   }
   float s;
   if (a.qstatic != nullptr) {
@@ -947,13 +952,20 @@ __global__ __launch_bounds__(1024) void decode_attn_combine_quant_kernel(DecodeA
     if (!(s > 0.f)) s = 1.f;
   }
   if (threadIdx.x == 0) a.qscale[b] = s;
-  int8_t* qrow = a.qout + (int64_t)b * a.ldq;
+  auto codes = [&](int h, const float (&v)[DPL]) {
+    int8_t* qrow = a.qout + (int64_t)b * a.ldq + h * D + lane;
 #pragma unroll
-  for (int k = 0; k < HPW; ++k) {
-    const int h = wave + k * nw;
-    if (h < a.H) {
+    for (int q = 0; q < DPL; ++q) qrow[64 * q] = ll_quant1(v[q], s);
+  };
+  if constexpr (HPW > 0) {
 #pragma unroll
-      for (int q = 0; q < DPL; ++q) qrow[h * D + lane + 64 * q] = ll_quant1(y[k][q], s);
+    for (int k = 0; k < HPW; ++k)
+      if (wave + k * nw < a.H) codes(wave + k * nw, y[k]);
+  } else {
+    for (int h = wave; h < a.H; h += nw) {
+#pragma unroll
+      for (int q = 0; q < DPL; ++q) y[0][q] = ll_to_f32(out_of(h)[64 * q]);
+      codes(h, y[0]);
     }
   }
 }
@@ -1142,19 +1154,19 @@ void launch_split_stage(const DecodeArgs& a, int dtype, unsigned grid, size_t ld
   }
 }
 
+template <typename T, int D>
+void launch_combine_quant(const DecodeArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)a.B), block((unsigned)(64 * (a.H < 16 ? a.H : 16)));
+  if (a.H <= 16) hipLaunchKernelGGL((decode_attn_combine_quant_kernel<T, D, 1>), grid, block, 0, stream, a);
+  else if (a.H <= 32) hipLaunchKernelGGL((decode_attn_combine_quant_kernel<T, D, 2>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((decode_attn_combine_quant_kernel<T, D, 0>), grid, block, 0, stream, a);
+}
+
 template <int D>
 void launch_combine(const DecodeArgs& a, int dtype, hipStream_t stream) {
   if (a.qout != nullptr) {
-    const int nw = a.H < 16 ? a.H : 16;
-    const dim3 qgrid((unsigned)a.B), qblock((unsigned)(64 * nw));
-    const bool two = a.H > 16;
-    if (dtype == LL_BF16) {
-      if (two) hipLaunchKernelGGL((decode_attn_combine_quant_kernel<__bf16, D, 2>), qgrid, qblock, 0, stream, a);
-      else hipLaunchKernelGGL((decode_attn_combine_quant_kernel<__bf16, D, 1>), qgrid, qblock, 0, stream, a);
-    } else {
-      if (two) hipLaunchKernelGGL((decode_attn_combine_quant_kernel<_Float16, D, 2>), qgrid, qblock, 0, stream, a);
-      else hipLaunchKernelGGL((decode_attn_combine_quant_kernel<_Float16, D, 1>), qgrid, qblock, 0, stream, a);
-    }
+    if (dtype == LL_BF16) launch_combine_quant<__bf16, D>(a, stream);
+    else launch_combine_quant<_Float16, D>(a, stream);
     return;
   }
   const dim3 cgrid((unsigned)((a.B * a.H + kCombWaves - 1) / kCombWaves));

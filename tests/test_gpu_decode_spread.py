@@ -99,6 +99,59 @@ def test_spread_fused_rope_equals_separate(cuda, quant):
         assert torch.equal(qc, wq) and torch.equal(qs, ws)
 
 
+@pytest.mark.parametrize("B,H,KVH,D,bound,same_launch", [
+    (2, 40, 8, 128, 8192, True), (1, 64, 8, 128, 4096, True), (3, 33, 3, 64, 8192, True),
+    (8, 40, 8, 128, 600, False), (9, 64, 8, 64, 1000, False), (3, 32, 4, 128, 8192, True),
+    (4, 7, 1, 128, 4096, True)])
+def test_quantising_merge_in_a_second_launch_holds_any_head_count(cuda, B, H, KVH, D, bound,
+                                                                  same_launch):
+    """Heads on both sides of what the merging waves keep in registers (16 and
+    32), splits merged by the second launch because they are spread or because
+    the same-launch merge is off: equal to the separate scatter, attention and
+    quantiser bit for bit, the workspace left at zero."""
+    from lite_lang_amd import _lib
+    ops = _ops()
+    assert _lib.load().ll_decode_attention_split_count(B, KVH, D, bound) > (8 if same_launch else 1)
+    g = torch.Generator().manual_seed(64)
+    lens = [max(1, bound - b * 977) for b in range(B)]
+    W, P = (H + 2 * KVH) * D, B * bound
+    pool = torch.randn(P, 2 * KVH, D, generator=g).bfloat16().to(cuda)
+    r2t = torch.randperm(P, generator=g).view(B, bound).to(torch.int32).to(cuda)
+    cos = torch.randn(bound, D // 2, generator=g).clamp(-1, 1).to(cuda)
+    sin = torch.randn(bound, D // 2, generator=g).clamp(-1, 1).to(cuda)
+    bias = torch.randn(W, generator=g).bfloat16().to(cuda)
+    ln = torch.tensor(lens, dtype=torch.int32, device=cuda)
+    pos, rids = ln - 1, torch.arange(B, dtype=torch.int32, device=cuda)
+    slots = r2t[torch.arange(B, device=cuda), pos.long()].contiguous()
+    part = torch.randint(-4000, 4000, (2, B, W), generator=g, dtype=torch.int32).to(cuda)
+    st = (torch.rand(B, generator=g) * 0.01 + 1e-3).to(cuda)
+    sc = (torch.rand(W, generator=g) * 0.05 + 1e-3).bfloat16().to(cuda)
+    static = torch.tensor([0.03], device=cuda)
+    print(f"case: quantising merge B={B} H={H}/{KVH} D={D} bound={bound} {same_launch}", flush=True)
+    p2 = pool.clone()
+    qbuf = torch.empty(B, H * D, dtype=torch.bfloat16, device=cuda)
+    want = torch.empty(B, H, D, dtype=torch.bfloat16, device=cuda)
+    f = torch.empty(B, W, device=cuda)
+    ops.dequant_splitk(part.view(-1), 2, st, sc, f, B, W)
+    ops.rope_kv_scatter_splitk(f.view(-1), 1, bias, qbuf, H, KVH, D, pos, cos, sin, slots, p2)
+    ops.decode_attention(qbuf.view(B, H, D), r2t, rids, ln, bound, p2[:, :KVH], p2[:, KVH:], want)
+    prev = ops.set_same_launch_merge(same_launch)
+    try:
+        for scale in (None, static):
+            p1 = pool.clone()
+            out = torch.full((B, H, D), 9.0, dtype=torch.bfloat16, device=cuda)
+            _, qc, qs = ops.decode_attention_rope_splitk_i32(
+                ops.I8Partials(part.view(-1), 2, st, sc), bias, pos, cos, sin, slots, r2t, rids, ln,
+                bound, p1[:, :KVH], p1[:, KVH:], out, quant=True, input_scale=scale)
+            assert torch.equal(out, want) and torch.equal(p1, p2)
+            wq, ws = (ops.quant_per_token(want.view(B, H * D)) if scale is None
+                      else ops.quant_static(want.view(B, H * D), scale))
+            assert torch.equal(qc, wq) and torch.equal(qs, ws)
+            assert ops.workspace(cuda, "decode_attention", 0).count_nonzero() == 0
+    finally:
+        ops.set_same_launch_merge(prev)
+
+
 def test_split_plan_never_outgrows_one_xcd():
     """Host only: up to 16 splits from 8 (sequence, KV head) units up, and the
     workspace never larger than with one split per eight 16-token tiles."""
