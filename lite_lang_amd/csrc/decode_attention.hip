@@ -1096,35 +1096,66 @@ struct SplitPlan {
 // The split count, and whether a unit's splits stay on one XCD (whose split
 // stage merges up to kUnitMergeSplits of them itself) or are spread over all
 // (a few long sequences otherwise leave XCDs idle or give one of them several
-// rounds of workgroups) and merged by a second launch. Swept over 1-33
-// sequences of 1000-16384 tokens, us per call:
-// * more than kUnitMergeSplits splits are spread: 1 x 6001 tokens 26.1 with
-//   47 splits on one XCD, 13.3 with 16, 11.7 spread; 1 x 4096 20.8, 11.8,
-//   10.7; 3 x 12001 28 with 42, 19.6, 17.5; 4 x 8000 17.9 and 15.4; 12 x 2000
-//   17.5 and 12.5;
-// * up to that many only where a wave of the busiest CU takes at least three
-//   rounds of tiles less (about 2.5 us each, against 4.5 us for the launch);
-// * below 8 units at most 16 splits, or one per 24 tiles (1 x 8192: 12.7 with
-//   32, 13.1 with 16, 15.8 with 64; 1 x 16384: 16.0, 19.0, 17.5), and none
-//   that saves no round of tiles (1 x 1000: 8.5 with 4, 9.8 with 7).
+// rounds of workgroups) and merged by a second launch. From a sweep of counts
+// and both forms over 1-20 sequences of 300-16000 tokens with 2, 4 and 8 KV
+// heads of 128 and 64, captured in a graph, us per call (q heads / KV heads of
+// 128 unless said):
+// * the same-launch merge loads the rows of up to 4, or of 8 splits at once, the
+//   second launch of 4, 8 or 16: a count between pays for the next one. Up to
+//   71 tiles 4 same-launch splits (1 x 1100 tokens, 16/2: 8.5; with 5 10.2, 8
+//   9.5; 4 x 1000, 32/8: 10.0, with 8 14.1), up to 127 tiles 8 spread (1 x 1500,
+//   16/2: 8.3; 6 same-launch 10.4, 11 spread 9.3), beyond it 16 (1 x 3000: 9.3;
+//   12 spread 10.1);
+// * more than 16 only below 8 units or at head_dim 64, one per 24 tiles in
+//   sixteens (1 x 16000, 16/2: 32 15.5, 16 18.3, 64 17.6; 4 x 6000, 8/2 heads
+//   of 64: 16 10.2, 42 13.5);
+// * up to 7 splits are spread only where a wave of the busiest CU takes at
+//   least three rounds of tiles less for it (12 x 2048, 28/4: 5 splits 20.9 ->
+//   15.8).
+// head_dim 64 has half the bytes per token and two workgroups per CU, so that
+// the second launch pays later, and not at all where the XCDs carry equal
+// loads or the stream from HBM is the bound:
+// * up to 191 tiles the same-launch merge of 8, where it fills at most three
+//   quarters of an XCD (1 x 2500, 8/2: 7.8, 16 spread 8.0; 16 x 1500: 8.2,
+//   spread 10.5);
+// * at any length with a multiple of 8 sequences (16 x 8192, 8/2: 17.0, 16
+//   spread 19.3), and for many units of 72 MB of K/V in all (6 x 8192, 32/8:
+//   27.3, 10 spread 29.5; 20 x 2048: 22.7 and 24.1; but 12 x 4096 runs 28.5
+//   spread and 27.2 not, which would cost it 1.4 where contexts are far below
+//   the bound, and stays spread).
 // No shape takes more splits than one XCD would give it (the workspace does
 // not grow).
 SplitPlan choose_splits(int B, int KVH, int64_t max_len, int64_t head_dim) {
   int ns = choose_nsplit_xcd(B, KVH, max_len, head_dim);
-  const int units = B * KVH;
+  const int units = B * KVH, seqs = (B + 7) / 8;  // sequences of the busiest XCD
   const int64_t tiles = (max_len + kTT - 1) / kTT;
   const int min_ns = (int)((tiles * kTT + kMaxSplitTokens - 1) / kMaxSplitTokens);
-  auto tile_rounds = [&](int n) { return ll_cdiv((tiles + n - 1) / n, kWaves); };
-  if (units < 8 && ns > 1) {
-    ns = std::max(min_ns, std::min(ns, std::max(16, (int)(tiles / 24))));
-    ns = std::max(min_ns, ll_cdiv(tiles, kWaves * tile_rounds(ns)));
+  const bool d64 = head_dim == 64;
+  if (units < 8 || d64) ns = std::min(ns, std::max(16, (int)(tiles / 24) / 16 * 16));
+  if (tiles < 72 && (units < 64 || d64)) ns = std::min(ns, 4);
+  const bool eight = tiles >= 72 && tiles < 128 && units < 64;
+  if (eight && ns < 16) ns = std::min(ns, kUnitMergeSplits);
+  ns = std::max(ns, std::max(min_ns, 1));
+  const bool even = d64 && (seqs * 8 == B ||
+                            (units >= 48 && 2 * seqs * 8 < 3 * B &&
+                             (ns >= kUnitMergeSplits || 4 * seqs * 8 <= 5 * B) &&
+                             B * tiles * kTT * KVH * 64 * 4 >= 72000000));
+  if (d64 && ns >= kUnitMergeSplits &&
+      (even || (tiles < 192 && seqs * KVH * kUnitMergeSplits <= 48))) {
+    ns = std::max(kUnitMergeSplits, min_ns);
+    return {ns, ns > kUnitMergeSplits};
   }
-  if (ns > kUnitMergeSplits) return {ns, true};
+  if (ns > kUnitMergeSplits || (ns == kUnitMergeSplits && (d64 || eight))) return {ns, true};
   const int per_cu = split_wg_per_cu(head_dim);
-  const int64_t xcd_wgs = (int64_t)((B + 7) / 8) * KVH * ns;
+  const int64_t xcd_wgs = (int64_t)seqs * KVH * ns;
   const int saved = (ll_cdiv(xcd_wgs, 32 * per_cu) - ll_cdiv((int64_t)units * ns, 256 * per_cu)) *
-                    tile_rounds(ns);
-  return {ns, ns > 1 && saved >= kSpreadRounds};
+                    ll_cdiv((tiles + ns - 1) / ns, kWaves);
+  return {ns, ns > 1 && !even && saved >= kSpreadRounds};
+}
+
+// workgroups of the split stage
+unsigned split_grid(int B, int KVH, const SplitPlan& p) {
+  return (unsigned)((p.spread ? B : (B + 7) / 8 * 8) * KVH * p.ns);
 }
 
 int64_t align256(int64_t x) { return ((x + 255) / 256) * 256; }
@@ -1233,9 +1264,7 @@ int launch_mfma(DecodeArgs& a, int64_t head_dim, int dtype, bool rope, int64_t m
   }
   const int64_t tiles = (max_len + kTT - 1) / kTT;
   a.slots_cap = (int)((tiles + a.nsplit - 1) / a.nsplit) * kTT;
-  const int groups = (a.B + 7) / 8;  // sequences per XCD
-  const unsigned grid = plan.spread ? (unsigned)(a.units * a.nsplit)
-                                    : (unsigned)(groups * 8 * a.KVH * a.nsplit);
+  const unsigned grid = split_grid(a.B, a.KVH, plan);
   const size_t extra = (size_t)a.slots_cap * 4 + (rope ? (size_t)(a.G + 2) * head_dim * 2 : 0);
   const int mode = !rope ? 0 : (!a.qkv.i32 && a.qkv.splits <= kRopeF32Splits) ? 1 : 2;
   if (head_dim == 128) {
@@ -1284,9 +1313,9 @@ extern "C" int ll_decode_attention_xcc_probe(int64_t batch, int64_t q_heads, int
   LL_CHECK_ARG(out != nullptr && batch > 0 && kv_heads > 0 && q_heads % kv_heads == 0 &&
                    (head_dim == 64 || head_dim == 128) && max_len_in_batch > 0,
                "ll_decode_attention_xcc_probe: bad arguments");
-  const int nsplit = choose_splits((int)batch, (int)kv_heads, max_len_in_batch, head_dim).ns;
-  const int groups = (int)((batch + 7) / 8);
-  const int64_t grid = (int64_t)groups * 8 * kv_heads * nsplit;
+  const SplitPlan plan = choose_splits((int)batch, (int)kv_heads, max_len_in_batch, head_dim);
+  const int nsplit = plan.ns;
+  const int64_t grid = split_grid((int)batch, (int)kv_heads, plan);
   LL_CHECK_ARG(out_len >= grid, "ll_decode_attention_xcc_probe: out holds %lld of %lld entries",
                (long long)out_len, (long long)grid);
   const int64_t tiles = (max_len_in_batch + kTT - 1) / kTT;
@@ -1311,6 +1340,11 @@ extern "C" int ll_decode_attention_set_same_launch_merge(int enable) {
 extern "C" int ll_decode_attention_split_count(int64_t batch, int64_t kv_heads, int64_t head_dim,
                                                int64_t max_len_in_batch) {
   return choose_splits((int)batch, (int)kv_heads, max_len_in_batch, head_dim).ns;
+}
+
+extern "C" int ll_decode_attention_splits_spread(int64_t batch, int64_t kv_heads, int64_t head_dim,
+                                                 int64_t max_len_in_batch) {
+  return choose_splits((int)batch, (int)kv_heads, max_len_in_batch, head_dim).spread ? 1 : 0;
 }
 
 extern "C" int64_t ll_decode_attention_workspace_size(int64_t batch, int64_t q_heads,

@@ -158,7 +158,8 @@ def decode_attention_xcd_premise(device, batch, q_heads, kv_heads, head_dim, max
                                  launches=3):
     """Checks, on this machine, the premise of the split stage's own merge:
     the probe kernel runs on exactly the split stage's grid, block and LDS
-    size for this shape and reports every workgroup's XCD; the premise holds
+    size for this shape (also where its splits are spread and need no such
+    premise: other batches of the same model merge in the launch) and reports every workgroup's XCD; the premise holds
     when workgroups whose indices agree mod 8 ran on one XCD (the split stage
     gives every workgroup of a sequence indices of one residue), which the
     dispatcher's round-robin over 8 XCDs gives, and so does a device of one

@@ -1,0 +1,45 @@
+"""The split rule of decode attention (host-only queries): where its lines lie,
+and that no shape takes more splits than its workspace bound."""
+import pytest
+
+from lite_lang_amd import _lib
+
+
+def _plan(B, KVH, D, n):
+    L = _lib.load()
+    return (L.ll_decode_attention_split_count(B, KVH, D, n),
+            L.ll_decode_attention_splits_spread(B, KVH, D, n))
+
+
+@pytest.mark.parametrize("KVH,D", [(1, 128), (2, 128), (4, 128), (8, 128), (2, 64), (8, 64)])
+def test_split_counts_stay_within_their_bounds(KVH, D):
+    """At least what the slot table's LDS asks for; otherwise at most one split
+    per eight 16-token tiles and one dispatch round, at most 16 from 8
+    (sequence, KV head) units up at head_dim 128, at most 16 or one per 24 tiles
+    below 8 units and at head_dim 64. A same-launch merge holds 8."""
+    for B in (1, 2, 3, 4, 7, 8, 9, 16, 20, 33, 40, 64, 128, 300):
+        for n in list(range(1, 3300, 61)) + [4096, 12001, 70000, 140000]:
+            ns, spread = _plan(B, KVH, D, n)
+            tiles, units = -(-n // 16), B * KVH
+            low = max(1, -(-tiles * 16 // 4096))
+            cap = min(256 * (1 if D == 128 else 2) // units, tiles // 8)
+            if units >= 8 and D == 128:
+                cap = min(cap, 16)
+            else:
+                cap = min(cap, max(16, tiles // 24))
+            assert low <= ns <= max(low, cap), (B, n)
+            assert spread in (0, 1) and (spread or ns <= 8) and (not spread or ns > 1), (B, n)
+
+
+@pytest.mark.parametrize("B,KVH,D,n,ns,spread", [
+    (1, 2, 128, 600, 4, 0), (3, 2, 128, 450, 3, 0), (1, 2, 128, 1100, 4, 0),  # few tiles
+    (1, 2, 128, 1136, 4, 0), (1, 2, 128, 1137, 8, 1), (2, 2, 128, 1500, 8, 1),
+    (1, 2, 128, 2032, 8, 1), (1, 2, 128, 2033, 16, 1), (1, 4, 128, 2500, 16, 1),
+    (3, 2, 128, 12001, 16, 1), (1, 2, 128, 16000, 32, 1),
+    (4, 8, 128, 1000, 4, 0), (4, 8, 128, 1500, 8, 1), (40, 2, 128, 600, 2, 0),
+    (1, 2, 64, 2500, 8, 0), (1, 2, 64, 3057, 16, 1), (16, 2, 64, 1500, 8, 0),
+    (16, 2, 64, 8192, 8, 0), (4, 2, 64, 8192, 16, 1), (1, 8, 64, 1300, 8, 1),
+    (6, 8, 64, 8192, 8, 0), (20, 8, 64, 2048, 3, 0), (10, 8, 64, 4096, 6, 1),
+    (12, 8, 64, 4096, 5, 1), (12, 8, 64, 1024, 4, 0)])
+def test_split_rule(B, KVH, D, n, ns, spread):
+    assert _plan(B, KVH, D, n) == (ns, spread)

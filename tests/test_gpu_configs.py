@@ -306,9 +306,11 @@ def test_decode_attention_xcd_premise(cuda, shape):
     the whole launch (decode_attention.hip map_block gives all splits of a
     sequence indices of one residue mod 8). r itself is not fixed: the
     round-robin continues from the previous launch. The probe reads XCC_ID on
-    exactly that grid, block and LDS size, several launches in a row."""
+    exactly that grid, block and LDS size, several launches in a row; every
+    shape here merges in the same launch (or needs no merge)."""
     from lite_lang_amd import _lib
     L = _lib.load()
+    assert L.ll_decode_attention_splits_spread(shape[0], *shape[2:]) == 0
     out = torch.full((1 << 14,), -1, dtype=torch.int32, device=cuda)
     print(f"case: xcc probe {shape}", flush=True)
     rotations = set()

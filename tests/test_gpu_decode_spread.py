@@ -40,8 +40,13 @@ def _run(cuda, q, pool, r2t, lens, KVH, bound):
 @pytest.mark.parametrize("B,H,KVH,D,L,dtype", [
     (1, 16, 2, 128, 4096, torch.bfloat16), (1, 12, 2, 128, 6001, torch.float16),
     (3, 16, 2, 128, 2500, torch.bfloat16), (2, 28, 4, 128, 3001, torch.float16),
-    (9, 12, 2, 128, 2200, torch.bfloat16), (2, 8, 2, 64, 5000, torch.bfloat16)])
+    (9, 12, 2, 128, 2200, torch.bfloat16), (2, 8, 2, 64, 5000, torch.bfloat16),
+    (1, 16, 2, 128, 1500, torch.bfloat16), (1, 32, 8, 64, 1300, torch.float16),
+    (10, 16, 8, 64, 1800, torch.bfloat16)])
 def test_spread_splits_match_oracle(cuda, B, H, KVH, D, L, dtype):
+    from lite_lang_amd import _lib
+    assert _lib.load().ll_decode_attention_splits_spread(B, KVH, D, L) == 1
+    assert _lib.load().ll_decode_attention_splits_spread(2, KVH, D, 300) == 0
     lens = [max(1, L - (b * 1237) % L) for b in range(B)]
     lens[-1] = min(lens[-1], 40) if B > 1 else lens[-1]  # most splits of one sequence are empty
     q, pool, r2t = _case(B, H, KVH, D, lens, dtype, 61)
@@ -64,6 +69,8 @@ def test_spread_fused_rope_equals_separate(cuda, quant):
     r2t = torch.randperm(7000, generator=g)[:2 * 3500].view(2, 3500).to(torch.int32)
     r2t = torch.cat([r2t, r2t.flip(0)], 1).to(cuda)  # rows of 7000 entries
     lens = [3400, 17]
+    from lite_lang_amd import _lib
+    assert _lib.load().ll_decode_attention_splits_spread(B, KVH, D, bound) == 1
     W = (H + 2 * KVH) * D
     cos = torch.randn(bound, D // 2, generator=g).clamp(-1, 1).to(cuda)
     sin = torch.randn(bound, D // 2, generator=g).clamp(-1, 1).to(cuda)
@@ -110,8 +117,10 @@ def test_quantising_merge_in_a_second_launch_holds_any_head_count(cuda, B, H, KV
     the same-launch merge is off: equal to the separate scatter, attention and
     quantiser bit for bit, the workspace left at zero."""
     from lite_lang_amd import _lib
+    L = _lib.load()
     ops = _ops()
-    assert _lib.load().ll_decode_attention_split_count(B, KVH, D, bound) > (8 if same_launch else 1)
+    assert L.ll_decode_attention_split_count(B, KVH, D, bound) > 1
+    assert L.ll_decode_attention_splits_spread(B, KVH, D, bound) == same_launch
     g = torch.Generator().manual_seed(64)
     lens = [max(1, bound - b * 977) for b in range(B)]
     W, P = (H + 2 * KVH) * D, B * bound
@@ -150,16 +159,3 @@ def test_quantising_merge_in_a_second_launch_holds_any_head_count(cuda, B, H, KV
             assert ops.workspace(cuda, "decode_attention", 0).count_nonzero() == 0
     finally:
         ops.set_same_launch_merge(prev)
-
-
-def test_split_plan_never_outgrows_one_xcd():
-    """Host only: up to 16 splits from 8 (sequence, KV head) units up, and the
-    workspace never larger than with one split per eight 16-token tiles."""
-    from lite_lang_amd import _lib
-    L = _lib.load()
-    for B in (1, 2, 3, 4, 7, 9, 20, 40, 64):
-        for n in (1, 16, 600, 1000, 4096, 12001, 70000, 140000):
-            ns = L.ll_decode_attention_split_count(B, 2, 128, n)
-            tiles = -(-n // 16)
-            low = -(-tiles * 16 // 4096)
-            assert max(1, low) <= ns <= max(1, low, min(max(1, 128 // B), tiles // 8 or 1))

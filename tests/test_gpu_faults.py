@@ -247,13 +247,17 @@ def test_split_merge_fallback_equals_same_launch(cuda, shape):
     """The runner's fallback when the XCD premise fails: with the same-launch
     merge switched off, decode attention merges its splits in a separate
     kernel; the outputs equal the same-launch merge's bit for bit (same
-    partials, same combine arithmetic)."""
+    partials, same combine arithmetic). Both shapes merge 2 to 8 splits in the
+    same launch by default."""
+    from lite_lang_amd import _lib
     ops = _ops()
     B, H, KVH, D, lens = shape
     rs = np.random.RandomState(6)
     if lens is None:
         lens = rs.randint(1, 3000, size=B).tolist()
     max_len = max(lens)
+    assert 2 <= _lib.load().ll_decode_attention_split_count(B, KVH, D, max_len) <= 8
+    assert _lib.load().ll_decode_attention_splits_spread(B, KVH, D, max_len) == 0
     P = B * max_len
     g = torch.Generator(device=cuda).manual_seed(6)
     q = torch.randn(B, H, D, device=cuda, generator=g).bfloat16()

@@ -83,8 +83,8 @@ def test_decode_attention_config2_varlen(cuda):
 def test_decode_attention_split_counts(cuda, B, L, splits):
     """Shapes on either side of the split-count rule (head_dim 128): at most
     16 splits from 8 (sequence, KV head) units up (4 x 8000 tokens would
-    fill a dispatch round with 32, 7 x 3000 with 18; more than 8 splits merge
-    by ticket), and from 64 units up the count the cost fit picks (2 splits
+    fill a dispatch round with 32, 7 x 3000 with 18; more than 8 splits are
+    spread over the XCDs and merge in a second launch), and from 64 units up the count the cost fit picks (2 splits
     at 32 x 600, 3 at 40 x 656). Each against the oracle."""
     from lite_lang_amd import _lib
     assert _lib.load().ll_decode_attention_split_count(B, 2, 128, L) == splits
