@@ -15,9 +15,12 @@ decode forward for a fixed batch size is captured once into a HIP graph:
   * the argmax writes the next tokens straight into the static token buffer
     the embedding of the next replay reads, so consecutive steps chain on the
     device without a host round trip;
-  * decode attention is captured with the runner's max_length as the length
-    bound: its split count and workspace are fixed, and every sequence
-    divides its own current length among the splits (ll_decode_attention).
+  * decode attention is captured with a length bound: its split count and
+    workspace are fixed, and every sequence divides its own current length
+    among the splits (ll_decode_attention). The bound is the runner's
+    max_length, and for small batches, whose plan at that bound pays a second
+    (merge) launch per layer, a shorter one too (decode_bounds): a step replays
+    the smallest that holds its lengths.
 Every decode graph of a device is captured on one stream of this module's
 (_capture_stream), and the library workspaces that stream uses are reserved
 on it before capture, so nothing is allocated by the library inside the
@@ -62,6 +65,25 @@ def reserve_model_workspaces(model, batch, max_len):
             ops.reserve_workspace(model.device, "decode_epoch", 4)
 
 
+def decode_bounds(model, batch, max_len):
+    """Length bounds a decode step of `batch` is captured for, ascending: max_len,
+    and where decode attention's splits are spread at that bound (merged by a
+    launch of their own, which contexts far below the bound pay for nothing),
+    the largest power of two whose plan merges in the same launch. Fused RoPE
+    attention of 1 to 3 sequences of 100 tokens, 12/2 heads of 128, in a graph:
+    9.0-9.3 us at a bound of 2048, 7.1-7.2 at 1024."""
+    cfg = model.cfg
+    shape = (batch, cfg.num_key_value_heads, cfg.head_dim)
+    spread = _lib.load().ll_decode_attention_splits_spread
+    if (cfg.head_dim not in (64, 128) or model.dtype == torch.float32
+            or not spread(*shape, max_len)):
+        return [max_len]
+    short = 1 << (max_len - 1).bit_length() - 1  # the largest below max_len
+    while short and spread(*shape, short):
+        short >>= 1
+    return [short, max_len] if short >= 256 else [max_len]
+
+
 _CAPTURE_STREAMS: dict[int, torch.cuda.Stream] = {}
 
 
@@ -98,11 +120,15 @@ class DecodeGraph:
                 reserve_model_workspaces(model, b, max_len)
         # the slot table must never be written by the capture itself
         torch.cuda.synchronize(dev)
-        self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph, stream=stream):
-            model.decode_tokens(self.ids, self.meta[3], self.meta[4], self.meta[1], self.meta[0],
-                                kv_cache, max_len, out=self.ids, slot_write=self.meta[0:3])
-        self.logits = model.last_logits  # the graph's own logits buffer
+        self._graphs = []  # (length bound, graph, its own logits buffer), bounds ascending
+        for bound in decode_bounds(model, batch_size, max_len):
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                model.decode_tokens(self.ids, self.meta[3], self.meta[4], self.meta[1],
+                                    self.meta[0], kv_cache, bound, out=self.ids,
+                                    slot_write=self.meta[0:3])
+            self._graphs.append((bound, graph, model.last_logits))
+        _, self.graph, self.logits = self._graphs[-1]
         torch.cuda.synchronize(dev)
 
     def run(self, in_ids: torch.Tensor, slots, rids, cols, positions, seq_len) -> torch.Tensor:
@@ -120,6 +146,9 @@ class DecodeGraph:
         self._host_ev[i] = ev
         if in_ids.data_ptr() != self.ids.data_ptr():
             self.ids.copy_(in_ids.view(-1))
+        if len(self._graphs) > 1:
+            short = self._graphs[0]
+            _, self.graph, self.logits = short if hm[4].max() <= short[0] else self._graphs[-1]
         self.graph.replay()
         self.model.last_logits = self.logits
         return self.ids

@@ -43,3 +43,20 @@ def test_split_counts_stay_within_their_bounds(KVH, D):
     (12, 8, 64, 4096, 5, 1), (12, 8, 64, 1024, 4, 0)])
 def test_split_rule(B, KVH, D, n, ns, spread):
     assert _plan(B, KVH, D, n) == (ns, spread)
+
+
+@pytest.mark.parametrize("batch,KVH,D,max_len,dtype,bounds", [
+    (1, 2, 128, 2048, "bfloat16", [1024, 2048]), (14, 2, 128, 2048, "bfloat16", [1024, 2048]),
+    (3, 2, 128, 1025, "float16", [1025]), (1, 2, 128, 1500, "float16", [1024, 1500]),
+    (2, 2, 64, 8192, "bfloat16", [2048, 8192]), (1, 2, 64, 2048, "bfloat16", [2048]),
+    (40, 2, 128, 4096, "bfloat16", [4096]), (1, 2, 128, 8192, "float32", [8192]),
+    (1, 2, 96, 8192, "bfloat16", [8192])])
+def test_decode_graph_bounds(batch, KVH, D, max_len, dtype, bounds):
+    """A second, shorter capture only where the plan at max_length pays a merge
+    launch that the shorter bound does not."""
+    import types
+    import torch
+    from lite_lang_amd.models.qwen2.decode_graph import decode_bounds
+    cfg = types.SimpleNamespace(num_key_value_heads=KVH, head_dim=D)
+    model = types.SimpleNamespace(cfg=cfg, dtype=getattr(torch, dtype))
+    assert decode_bounds(model, batch, max_len) == bounds
