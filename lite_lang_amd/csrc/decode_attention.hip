@@ -1265,6 +1265,10 @@ int launch_mfma(DecodeArgs& a, int64_t head_dim, int dtype, bool rope, int64_t m
   const int64_t tiles = (max_len + kTT - 1) / kTT;
   a.slots_cap = (int)((tiles + a.nsplit - 1) / a.nsplit) * kTT;
   const unsigned grid = split_grid(a.B, a.KVH, plan);
+  // two launches: no other call may come between them on this workspace
+  std::unique_lock<std::mutex> lock;
+  if (a.nsplit > 1 && a.merge_cnt == nullptr)
+    lock = std::unique_lock<std::mutex>(ll_workspace_mutex(workspace));
   const size_t extra = (size_t)a.slots_cap * 4 + (rope ? (size_t)(a.G + 2) * head_dim * 2 : 0);
   const int mode = !rope ? 0 : (!a.qkv.i32 && a.qkv.splits <= kRopeF32Splits) ? 1 : 2;
   if (head_dim == 128) {

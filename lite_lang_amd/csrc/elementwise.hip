@@ -22,6 +22,11 @@ void ll_set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
+std::mutex& ll_workspace_mutex(const void* ws) {
+  static std::mutex mu[64];
+  return mu[((uintptr_t)ws >> 8) % 64];
+}
+
 extern "C" const char* ll_last_error(void) { return g_err; }
 
 extern "C" int ll_version(void) { return LL_ABI_VERSION; }

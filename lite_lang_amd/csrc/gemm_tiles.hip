@@ -986,6 +986,7 @@ int launch_tiles_ws(const TileArgs& a, void* ws, int64_t ws_bytes, hipStream_t s
   pa.Y = ws;
   pa.ldy = a.N;
   pa.split_b = split_b;
+  std::lock_guard<std::mutex> lock(ll_workspace_mutex(ws));
   const int prc = launch_plan<T, TP, __is_same(T, int8_t) ? EPI_I32 : EPI_PART>(pa, plan, cus, stream);
   if (prc != LL_OK) return prc;
   hipLaunchKernelGGL((tile_reduce_kernel<TP, TO>), dim3((unsigned)ll_cdiv((int64_t)a.M * (a.N / 4), 256)),

@@ -9,6 +9,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <mutex>
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -55,6 +57,11 @@ void ll_set_error(const char* fmt, ...);
 // (ll_decode_sync_set_spin_limit: 0 = each wait's default, n > 0 = n polls,
 // -n = test mode: the wait never sees its data and gives up after n polls).
 int ll_decode_spin_setting();
+// Held over the launches of a call that hand data on in a caller's workspace
+// (one of 64 mutexes, by its address), so that calls of several threads on one
+// stream and workspace run one after another there, as they do where a call is
+// a single launch (elementwise.hip).
+std::mutex& ll_workspace_mutex(const void* ws);
 // CUs of the current device, cached per device (gemm_tiles.hip): the
 // persistent grids hold one workgroup per CU, each looping over its work.
 int ll_device_cus(int* cus_out);

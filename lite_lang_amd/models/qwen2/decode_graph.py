@@ -45,10 +45,11 @@ def reserve_decode_workspaces(cfg, batch, max_len, device):
               (2 * cfg.intermediate_size, cfg.hidden_size),
               (cfg.hidden_size, cfg.intermediate_size), (cfg.vocab_size, cfg.hidden_size)]
     ops.reserve_workspace(device, "gemm",
-                          max(max(L.ll_gemm_workspace_size(batch, n, k),
-                                  L.ll_gemm_tiles_workspace_size(batch, n, k, 1),
-                                  L.ll_gemm_tiles_workspace_size(batch, n, k, 2))
-                              for n, k in shapes))
+                          max(L.ll_gemm_workspace_size(batch, n, k) for n, k in shapes))
+    if batch > 64:
+        ops.reserve_workspace(device, "gemm_tiles",
+                              max(L.ll_gemm_tiles_workspace_size(batch, n, k, es)
+                                  for n, k in shapes for es in (1, 2)))
     ops.reserve_workspace(device, "argmax", L.ll_argmax_workspace_size(batch, cfg.vocab_size))
     ops.reserve_workspace(device, "lm_argmax", L.ll_gemm_packed_f32_argmax_workspace_size(
         batch, cfg.vocab_size, cfg.hidden_size))

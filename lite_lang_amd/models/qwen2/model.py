@@ -142,15 +142,15 @@ class Qwen2Model:
 
     def _proj_norm(self, h, x, weight, gamma, splits):
         """h += x @ weight^T, returns its RMSNorm: the product's k splits into
-        the GEMM workspace, finished by the norm. None where the product does
-        not split, or inside a capture whose workspace is smaller."""
+        the stream's "norm_part" workspace, finished by the norm. None where the
+        product does not split, or inside a capture whose workspace is smaller."""
         if splits <= 1:
             return None
         need = splits * h.numel() * 4
-        _, have = ops.optional_workspace(h.device, "gemm", need)
+        _, have = ops.optional_workspace(h.device, "norm_part", need)
         if have < need:
             return None
-        part = ops.workspace(h.device, "gemm", need)[:need].view(torch.float32)
+        part = ops.workspace(h.device, "norm_part", need)[:need].view(torch.float32)
         s = ops.gemm_tiles_splitk(x, weight, part)
         return ops.add_rmsnorm_splitk(h, part, s, gamma, self.cfg.rms_norm_eps)
 

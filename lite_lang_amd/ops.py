@@ -376,13 +376,16 @@ def gemm(x, w, bias=None, out=None):
     fields = [x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
               bias.data_ptr() if bias is not None else 0, out.data_ptr(), out.stride(0), M, N, K,
               dtype_code(x), 0, 0, 0, 0]
-    need = _call(_L.ll_call_gemm, _lib.GEMM_CALL, fields, "ll_gemm", "gemm", 11, x)
+    # (a buffer of its own above 64 rows: the library keeps the two launches of a
+    # split product together, not those of the weight-streaming GEMMs)
+    ws = "gemm" if M <= 64 else "gemm_tiles"
+    need = _call(_L.ll_call_gemm, _lib.GEMM_CALL, fields, "ll_gemm", ws, 11, x)
     if need:
         if M > 64 and torch.cuda.is_current_stream_capturing():
             fields[13] = 1  # nothing is allocated inside a capture: run with what there is
         else:
-            workspace(x.device, "gemm", need)
-        _call(_L.ll_call_gemm, _lib.GEMM_CALL, fields, "ll_gemm", "gemm", 11, x)
+            workspace(x.device, ws, need)
+        _call(_L.ll_call_gemm, _lib.GEMM_CALL, fields, "ll_gemm", ws, 11, x)
     return out
 
 
@@ -447,7 +450,7 @@ def gemm_i8_tiled(xq, s_tok, wq, s_ch, bias=None, out_dtype=torch.bfloat16, out=
     assert s_tok.dtype == torch.float32 and s_ch.numel() == N
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=xq.device)
-    ws_ptr, ws_n = optional_workspace(xq.device, "gemm",
+    ws_ptr, ws_n = optional_workspace(xq.device, "gemm_tiles",
                                       _L.ll_gemm_tiles_workspace_size(M, N, K, 1))
     rc = _L.ll_gemm_i8_tiled_ws(xq.data_ptr(), xq.stride(0), s_tok.data_ptr(), wq.data_ptr(),
                                 wq.stride(0), s_ch.data_ptr(), dtype_code(s_ch),
