@@ -196,7 +196,10 @@ class DeviceWeights:
     def __init__(self, cfg: Qwen2Config, sd: dict, dtype: torch.dtype, device, pack: bool = True,
                  quant: str = None):
         def dev(t):
-            return t.to(device=device, dtype=dtype).contiguous()
+            # (a tensor already there may be a view at any element of a larger
+            # buffer; the GEMMs read 16-byte aligned rows)
+            t = t.to(device=device, dtype=dtype).contiguous()
+            return t if t.data_ptr() % 16 == 0 else t.clone()
 
         self.embed = dev(sd["model.embed_tokens.weight"])
         self.norm = dev(sd["model.norm.weight"])
