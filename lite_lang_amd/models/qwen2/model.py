@@ -254,11 +254,12 @@ class Qwen2Model:
     def fused_decode_ok(self, batch):
         """Whether a decode step of `batch` runs the fused split-K layer: up to
         64 rows on the weight-streaming GEMMs, up to _WIDE_DECODE on the tile
-        GEMM's partials (not W8A8)."""
+        GEMM's partials (not W8A8, nor head dims that the RoPE + K/V scatter of
+        partials does not take)."""
         if self.dtype not in (torch.bfloat16, torch.float16) or not 0 < batch <= _WIDE_DECODE:
             return False
         return batch <= 64 or (
-            self.quant != "w8a8" and self.cfg.hidden_size <= 8192
+            self.quant != "w8a8" and self.cfg.hidden_size <= 8192 and self.cfg.head_dim % 8 == 0
             and all(ops.gemm_tiles_splitk_count(batch, n, k, self.dtype) > 0
                     for n, k in self._wide_shapes()))
 

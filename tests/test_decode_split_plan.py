@@ -60,3 +60,19 @@ def test_decode_graph_bounds(batch, KVH, D, max_len, dtype, bounds):
     cfg = types.SimpleNamespace(num_key_value_heads=KVH, head_dim=D)
     model = types.SimpleNamespace(cfg=cfg, dtype=getattr(torch, dtype))
     assert decode_bounds(model, batch, max_len) == bounds
+
+
+@pytest.mark.parametrize("heads,head_dim,wide", [(8, 16, True), (16, 128, True), (8, 20, False),
+                                                 (72, 128, False)])
+def test_wide_fused_decode_takes_only_what_its_kernels_take(heads, head_dim, wide):
+    """Batches of 65 to 256 leave the general layer only where every kernel of
+    the fused one takes the shape: head_dim % 8 for the scatter of partials,
+    hidden <= 8192 for the norm."""
+    import torch
+    from lite_lang_amd.models.qwen2.model import Qwen2Model
+    from lite_lang_amd.models.qwen2.weights import Qwen2Config
+    cfg = Qwen2Config(layer_nums=1, hidden_size=heads * head_dim, num_heads=heads,
+                      num_key_value_heads=heads // 4, intermediate_size=256, vocab_size=32)
+    assert cfg.head_dim == head_dim
+    m = Qwen2Model(1, 64, cfg, 0, 1, torch.bfloat16, torch.device("cpu"))
+    assert [m.fused_decode_ok(b) for b in (64, 65, 256, 257)] == [True, wide, wide, False]
