@@ -258,6 +258,13 @@ int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t ldw, const 
  * int8); 0 where they do not split. With less they run one split. */
 int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K, int64_t elem_bytes);
 
+/* The tile GEMM's plan for a shape on 256 CUs (host only): output tile of
+ * tile_n weight rows x tile_m activation rows, k splits (split 0: one, as for
+ * the forms that take no workspace) and 128-byte K stages per split, the last
+ * split holding the rest. */
+int ll_gemm_tiles_plan(int64_t M, int64_t N, int64_t K, int64_t elem_bytes, int split,
+                       int32_t* tile_n, int32_t* tile_m, int32_t* splits, int32_t* split_stages);
+
 /* fp32 partial sums [splits][M][N] of the tile GEMM's product (bf16/fp16, the
  * layout rules of ll_gemm_tiled), for the split-K consumers (ll_add_rmsnorm_splitk,
  * ll_rope_kv_scatter_splitk, ll_decode_attention_rope_splitk). The split count

@@ -63,6 +63,7 @@ SIGNATURES = {
     "ll_gemm_gate_up_silu_tiled": (I32, [P, I64, P, I64, I64, I64, I32, P, I64, P]),
     "ll_gemm_i8_tiled": (I32, [P, I64, P, P, I64, P, I32, P, P, I64, I64, I64, I64, I32, P]),
     "ll_gemm_tiles_workspace_size": (I64, [I64, I64, I64, I64]),
+    "ll_gemm_tiles_plan": (I32, [I64, I64, I64, I64, I32, P, P, P, P]),
     "ll_gemm_tiles_splitk_count": (I32, [I64, I64, I64, I32]),
     "ll_gemm_tiles_splitk": (I32, [P, I64, P, I64, I64, I64, I64, I32, P, I64, P]),
     "ll_gemm_i8_tiled_ws": (I32, [P, I64, P, P, I64, P, I32, P, P, I64, I64, I64, I64, I32, P, I64,

@@ -1087,6 +1087,23 @@ extern "C" int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K,
   return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
 }
 
+extern "C" int ll_gemm_tiles_plan(int64_t M, int64_t N, int64_t K, int64_t elem_bytes, int split,
+                                  int32_t* tile_n, int32_t* tile_m, int32_t* splits,
+                                  int32_t* split_stages) {
+  LL_CHECK_ARG(tile_n && tile_m && splits && split_stages, "ll_gemm_tiles_plan: null pointer");
+  LL_CHECK_ARG(M > 0 && N > 0 && N % 4 == 0 && K > 0 && (elem_bytes == 1 || elem_bytes == 2) &&
+                   (K * elem_bytes) % kKUnit == 0,
+               "ll_gemm_tiles_plan: no tile GEMM of this shape (M=%lld N=%lld K=%lld)",
+               (long long)M, (long long)N, (long long)K);
+  const TilePlan p =
+      plan_tiles(M, N, K * elem_bytes, (int)elem_bytes, split ? kPlanCus : 1, kPlanCus);
+  *tile_n = p.geo == 2 ? 128 : 256;
+  *tile_m = p.geo == 0 ? 256 : 128;
+  *splits = p.splits;
+  *split_stages = p.kps;
+  return LL_OK;
+}
+
 // fp32 partial sums for a consumer that finishes them itself: a reduction
 // launch (4.5 us and the partials' bytes once more) less per product. Decode
 // step of 96 requests (4 layers, 3B): 570 -> 520 us; first token of one prompt

@@ -7,6 +7,8 @@ computes on the host; a missing library raises at import.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -540,6 +542,14 @@ def gemm_splitk(x, w, part):
                            dtype_code(x), part.data_ptr(), part.numel() * 4, _stream(x))
     _lib.check(rc, "ll_gemm_splitk")
     return s
+
+
+def gemm_tiles_plan(M, N, K, elem_bytes=2, split=True):
+    """(tile_n, tile_m, k splits, stages per split) of the tile GEMM for a shape."""
+    out = [ctypes.c_int32() for _ in range(4)]
+    rc = _L.ll_gemm_tiles_plan(M, N, K, elem_bytes, int(split), *map(ctypes.addressof, out))
+    _lib.check(rc, "ll_gemm_tiles_plan")
+    return tuple(v.value for v in out)
 
 
 def gemm_tiles_splitk_count(M, N, K, dtype) -> int:

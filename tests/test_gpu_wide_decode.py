@@ -39,8 +39,9 @@ def test_partials_sum_to_the_product(cuda, M, N, K, dtype):
         ops.gemm_tiles_splitk(x, w, part[:n * M * N - 4])
 
 
-def _steps(cuda, B, dtype, graph, head_dim, n_steps=2):
-    """Logits of a prefill of B short prompts and of the decode steps after it."""
+def _steps(cuda, B, dtype, graph, head_dim, n_steps=2, tokens=None):
+    """Logits and tokens of a prefill of B short prompts and of the decode steps
+    after it, which are fed the run's own tokens or the given ones."""
     from lite_lang_amd.models.qwen2 import Qwen2ModelRunner
     from lite_lang_amd.models.runner_batch import RunnerBatch
     cfg = Qwen2Config(layer_nums=3, hidden_size=4 * head_dim, num_heads=4, num_key_value_heads=2,
@@ -54,28 +55,30 @@ def _steps(cuda, B, dtype, graph, head_dim, n_steps=2):
                          use_cuda_graph=graph)
     r.init_model()
     batch = RunnerBatch.create_batch(msgs, "wide", True, r)
-    logits = []
-    for _ in range(1 + n_steps):
+    logits, outs = [], []
+    for i in range(1 + n_steps):
         out = r.forward(batch)
         logits.append(r.model_ins_.last_logits.float().clone())
-        batch.update_forward_message(out)
-    return r, logits
+        outs.append(out.clone())
+        batch.update_forward_message(out if tokens is None else tokens[i])
+    return r, logits, outs
 
 
 @pytest.mark.parametrize("B,dtype,graph,head_dim", [
     (65, torch.bfloat16, True, 128), (96, torch.float16, False, 128),
-    (128, torch.bfloat16, True, 64), (257, torch.float16, True, 64)])
+    (128, torch.bfloat16, True, 64), (129, torch.bfloat16, True, 128),  # two row tiles from 129
+    (160, torch.float16, True, 64), (256, torch.float16, False, 128),
+    (257, torch.float16, True, 64)])
 def test_wide_decode_matches_general_layer(cuda, monkeypatch, B, dtype, graph, head_dim):
     from lite_lang_amd.models.qwen2 import model
     print(f"case: wide decode B={B} {dtype} graph={graph} D={head_dim}", flush=True)
-    r, got = _steps(cuda, B, dtype, graph, head_dim)
+    r, got, toks = _steps(cuda, B, dtype, graph, head_dim)
     assert r.model_ins_.fused_decode_ok(B) == (B <= model._WIDE_DECODE)
     assert r.model_ins_._norm_splits(5 * B)[1] > 1  # the prefill's down_proj splits
     monkeypatch.setattr(model, "_WIDE_DECODE", 64)
     monkeypatch.setattr(model.Qwen2Model, "_norm_splits", lambda self, T: (1, 1))
-    _, want = _steps(cuda, B, dtype, graph, head_dim)
-    same = torch.ones(B, dtype=torch.bool, device=cuda)  # requests fed the same tokens so far
-    for a, b in zip(got, want):
-        assert float((a - b)[same].abs().max()) <= 2e-2
-        same &= a.argmax(-1) == b.argmax(-1)
-    assert same.float().mean() > 0.5
+    _, want, _ = _steps(cuda, B, dtype, graph, head_dim, tokens=toks)
+    for a, b, t in zip(got, want, toks):
+        assert float((a - b).abs().max()) <= 2e-2
+        # the picked tokens: the largest logit of either run but for a tie within the bar
+        assert float((b.amax(-1) - b.gather(-1, t).squeeze(-1)).max()) <= 4e-2
