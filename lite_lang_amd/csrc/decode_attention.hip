@@ -1265,9 +1265,11 @@ int launch_mfma(DecodeArgs& a, int64_t head_dim, int dtype, bool rope, int64_t m
   const int64_t tiles = (max_len + kTT - 1) / kTT;
   a.slots_cap = (int)((tiles + a.nsplit - 1) / a.nsplit) * kTT;
   const unsigned grid = split_grid(a.B, a.KVH, plan);
-  // two launches: no other call may come between them on this workspace
+  // No other thread's call may come between the split stage and its merge
+  // kernel on this workspace, one that merges in its own launch neither: it
+  // would take the partial words there for its own.
   std::unique_lock<std::mutex> lock;
-  if (a.nsplit > 1 && a.merge_cnt == nullptr)
+  if (a.nsplit > 1)
     lock = std::unique_lock<std::mutex>(ll_workspace_mutex(workspace));
   const size_t extra = (size_t)a.slots_cap * 4 + (rope ? (size_t)(a.G + 2) * head_dim * 2 : 0);
   const int mode = !rope ? 0 : (!a.qkv.i32 && a.qkv.splits <= kRopeF32Splits) ? 1 : 2;

@@ -22,23 +22,30 @@ def _gemm_i8(ops, g, cuda):
     return lambda: ops.gemm_i8_tiled(x, st, w, sc)
 
 
-def _attention(ops, g, cuda):
+def _attention(ops, g, cuda, n=3000):
     q = torch.randn(1, 12, 128, generator=g).bfloat16().to(cuda)
-    pool = torch.randn(3000, 4, 128, generator=g).bfloat16().to(cuda)
-    r2t = torch.randperm(3000, generator=g).to(torch.int32).view(1, -1).to(cuda)
+    pool = torch.randn(n, 4, 128, generator=g).bfloat16().to(cuda)
+    r2t = torch.randperm(n, generator=g).to(torch.int32).view(1, -1).to(cuda)
     rid = torch.zeros(1, dtype=torch.int32, device=cuda)
-    n = torch.tensor([3000], device=cuda)
-    return lambda: ops.decode_attention(q, r2t, rid, n, 3000, pool[:, :2], pool[:, 2:],
+    ln = torch.tensor([n], device=cuda)
+    return lambda: ops.decode_attention(q, r2t, rid, ln, n, pool[:, :2], pool[:, 2:],
                                         torch.empty_like(q))
 
 
-@pytest.mark.parametrize("make", [_gemm, _gemm_i8, _attention])
+def _attention_mixed(ops, g, cuda):
+    """The second thread's splits merge in their own launch."""
+    return _attention(ops, g, cuda, 1000 if g.initial_seed() % 3 == 0 else 3000)
+
+
+@pytest.mark.parametrize("make", [_gemm, _gemm_i8, _attention, _attention_mixed])
 def test_threads_on_one_stream(cuda, make):
     from lite_lang_amd import _lib, ops
     L = _lib.load()
     assert L.ll_gemm_tiles_workspace_size(96, 512, 4096, 2) > 0
     assert L.ll_gemm_tiles_workspace_size(96, 512, 4096, 1) > 0
     assert L.ll_decode_attention_splits_spread(1, 2, 128, 3000) == 1
+    assert L.ll_decode_attention_splits_spread(1, 2, 128, 1000) == 0
+    assert L.ll_decode_attention_split_count(1, 2, 128, 1000) > 1
     print(f"case: threads {make.__name__}", flush=True)
     calls = [make(ops, torch.Generator().manual_seed(98 + i), cuda) for i in range(3)]
     want = [c() for c in calls]
