@@ -255,7 +255,10 @@ int ll_gemm_tiled(const void* X, int64_t ldx, const void* W, int64_t ldw, const 
 
 /* Workspace with which ll_gemm (M > 64) and ll_gemm_i8_tiled_ws split the K of
  * a product with few output tiles over the CUs (elem_bytes 2: bf16/fp16, 1:
- * int8); 0 where they do not split. With less they run one split. */
+ * int8); 0 where they do not split. With less they run fewer splits or one.
+ * The split count follows M (and the workspace), and bf16/fp16 sums are taken
+ * in split order: a row's last bits can depend on how many rows share its call
+ * and, inside a captured graph, on the workspace there when it was captured. */
 int64_t ll_gemm_tiles_workspace_size(int64_t M, int64_t N, int64_t K, int64_t elem_bytes);
 
 /* The tile GEMM's plan for a shape on 256 CUs (host only): output tile of

@@ -5,15 +5,15 @@
 // (the reference's SmoothQuant module has no forward, quantize/smooth_quant/
 // layer.py:19-59).
 //
-// One workgroup (8 waves, two per SIMD) per CU works off (k split, output
-// tile) items one after the other (a persistent grid); tiles are 256 x 256,
-// 256 x 128 or 128 x 128 by shape (plan_tiles):
+// One workgroup per CU works off (k split, output tile) items one after the
+// other (a persistent grid); tiles are 256 x 256 or 256 x 128 (8 waves, two per
+// SIMD) or 128 x 128 (4 waves) by shape (plan_tiles):
 //   * stages of 128 bytes of K per row (64 bf16/fp16 or 128 int8) of the
 //     tile's weight and activation rows are copied global -> LDS with
 //     global_load_lds_dwordx4 (no VGPR staging) into a ring of two to four
 //     stage buffers that runs on from one item into the next. A row's 128
-//     bytes are one cache line: 64-byte rows fetched every line twice and
-//     fed a CU at 56 GB/s with all CUs reading, 128-byte rows at 134 GB/s;
+//     bytes are one cache line (with 64-byte rows every line was fetched
+//     twice);
 //   * the ring is refilled in pieces of 128 rows, each as soon as both wave
 //     groups have read it, so the copies lead the reads by more than a stage
 //     although the 256 x 256 form holds only two stages;
@@ -26,16 +26,19 @@
 //     with v_mfma_f32_16x16x32 (v_mfma_i32_16x16x64_i8 for int8) as
 //     C^T = W . X^T: the weight rows are the MFMA's row operand, so every
 //     lane ends with runs of 4 consecutive output columns of one token row.
-//     At large sizes the card is power-bound (1.6 GHz, the matrix pipes busy
-//     85% of the cycles), and the 16 x 16 form, which moves half the
-//     accumulator registers per product, runs 6% faster than 32 x 32;
+//     At 24,000 rows the matrix pipes are busy 63% of the cycles at about
+//     1.96 GHz (gate/up + SiLU; the 32 x 32 form with 64-byte rows: 69% at
+//     1.55 GHz): the 16 x 16 form, which moves half the accumulator registers
+//     per product, draws less and clocks higher, 6% faster than 32 x 32;
 //   * the grid is XCD-aware: the workgroups the dispatcher deals to one XCD
 //     take a contiguous range of items, tiles in groups of 1, 2 or 4 row
 //     tiles by shape (tile_group_m), round robin, so tiles sharing activation
 //     or weight rows run together on one L2.
-// Measured (bf16, one launch): gate/up + SiLU at M = 24,000 (3B) 1790 -> 1736
-// us (1247 TFLOP/s), down_proj 930 -> 780 (1388), qkv 272 -> 202; down_proj
-// at M = 333 204 -> 33 us.
+// Measured against 256 x 256 tiles of 64-byte rows and 32 x 32 products (bf16,
+// M = 24,000, 3B, 20 launches, both on one card): gate/up + SiLU 1850 -> 1695 us
+// (1277 TFLOP/s), down_proj 931 -> 810 (1336), qkv 271 -> 240, o_proj 197 -> 173;
+// W8A8 1519 -> 962, 512 -> 415, 210 -> 138, 160 -> 109. down_proj at M = 333
+// 204 -> 33 us.
 // Epilogues: the model dtype with an optional bias; SiLU_and_Mul of a
 // gate/up weight interleaved in 64-row blocks (ll_gemm_interleave_gate_up),
 // with the rounding sequence of ll_silu_and_mul; int8 sums dequantised as
@@ -52,7 +55,7 @@ namespace {
 constexpr int kRB = 128;       // bytes of K per row per stage: one cache line
 constexpr int kKUnit = 64;     // K spans a multiple of this many bytes
 constexpr int kPlanCus = 256;   // CUs the workspace query plans for
-constexpr int kMinSplitStages = 6;  // stages a k split holds at least
+constexpr int kMinSplitStages = 6;  // stages per k split on average, at least (the last has the rest)
 constexpr int kPieceB = 128 * kRB;  // a piece: 128 rows of one operand (16 KB)
 
 // Tile geometry: NWP pieces of 128 weight rows by NXP pieces of 128
@@ -77,7 +80,8 @@ constexpr int kPieceB = 128 * kRB;  // a piece: 128 rows of one operand (16 KB)
 // split, where every weight byte is read once and would only push the
 // activations out of L2 (96 rows, cold weights): gate/up + SiLU 26.9 -> 25.4
 // us (22016 x 2048) and 21.0 -> 20.2 (17920 x 1536), lm_head 157 -> 152 and
-// 110 -> 102. With two row tiles, which share the weights through L2, it
+// 110 -> 102; int8 gate/up + SiLU 21.7 -> 20.9 and 18.9 -> 18.4 (2 to 5% over 65
+// to 128 rows). With two row tiles, which share the weights through L2, it
 // costs (160 rows, 151936 x 2048: 174 -> 204), and k splits lose too (2048 x
 // 11008: 19.0 -> 21.2; 1536 x 8960: 15.7 -> 18.2).
 template <int NWP_, int NXP_, bool NT_ = false> struct TileGeo {
@@ -806,12 +810,13 @@ __global__ void interleave_gate_up_kernel(const u32x4* __restrict__ W, int64_t l
   out[u] = W[src * ldw16 + c];
 }
 
-// Row tiles per group of the tile order, by shape class, as measured on the
-// 3B prefill projections at M = 24,000 (group sizes 1, 2, 4 and 8, libraries
-// interleaved, best of 4 rounds): wide outputs (gate/up, 86 column tiles)
-// 4 (1788 us against 1813 with 2 and 1886-1898 with 1 or 8); long K
-// (down_proj, 172 stages) 1 (916 against 953 with 2); the narrow short-K
-// shapes (qkv, o_proj) level at every size (2).
+// Row tiles per group of the tile order, by shape class, as measured with group
+// sizes 1, 2, 4 and 8 (us): wide outputs 4 (gate/up + SiLU, 86 column tiles, M =
+// 24,000: 1712, 1655, 1634, 1626; 256 x 128 tiles, M = 600: 70.5, 57.2, 56.4,
+// 55.3; lm_head of 1536, M = 600: 503, 327, 318, 300; the 8 of these lead the 4 by
+// 0.5 to 6%, but not at M = 8192: 565, 557, 546, 547); long K (down_proj, 172
+// stages, M = 24,000) 1 (773, 777, 791, 808); the narrow short-K shapes (qkv,
+// o_proj) level within 1.5% at every size (2).
 int tile_group_m(int64_t tiles_n, int64_t nk) {
   if (tiles_n >= 32) return 4;
   if (nk >= 64) return 1;
@@ -835,6 +840,11 @@ struct TilePlan {
 // in 5 splits, 98 unsplit, 197 as 16 tiles of 256 x 256), and what lies
 // between follows the rounds its tiles take (600 x 22016: 71 us in two
 // rounds of 256 x 128, 97 in two of 256 x 256).
+// The cost has no term for the weights' bytes: it says 95 us for the lm_head of
+// 96 rows, which streams 622 MB in 145 to 152. What it orders are forms of one
+// shape, which move the same bytes: with each form forced, its choice was within
+// 3% of the best for lm_head and gate/up at 65 to 600 rows, but for a 1536-wide
+// lm_head at 256 rows (152 us, best 145) and at 600 (327, best 302).
 // A K that ends in half a stage runs on the 256 x 256 form, the only one that
 // can leave out a k step; int8 has no 128 x 128 form (its sums and two
 // fragment sets do not fit the registers).
@@ -1106,7 +1116,7 @@ extern "C" int ll_gemm_tiles_plan(int64_t M, int64_t N, int64_t K, int64_t elem_
 
 // fp32 partial sums for a consumer that finishes them itself: a reduction
 // launch (4.5 us and the partials' bytes once more) less per product. Decode
-// step of 96 requests (4 layers, 3B): 570 -> 520 us; first token of one prompt
+// step of 96 requests (4 layers, 3B): 570 -> 528 us; first token of one prompt
 // of 333 (4 layers): 749 -> 737.
 extern "C" int ll_gemm_tiles_splitk_count(int64_t M, int64_t N, int64_t K, int dtype) {
   if (!ll_gemm_tiled_supported(M, N, K, dtype)) return 0;
