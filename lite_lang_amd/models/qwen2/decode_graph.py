@@ -64,6 +64,8 @@ def reserve_model_workspaces(model, batch, max_len):
             ops.reserve_workspace(model.device, "w8a8_part", model.w8a8_part_bytes(batch))
         if model.norm_qkv_splits(batch) > 0:
             ops.reserve_workspace(model.device, "decode_epoch", 4)
+    elif model.norm_part_bytes(batch) > 0:  # the general layer's k-split o_proj and down_proj
+        ops.reserve_workspace(model.device, "norm_part", model.norm_part_bytes(batch))
 
 
 def decode_bounds(model, batch, max_len):

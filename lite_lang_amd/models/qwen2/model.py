@@ -140,6 +140,11 @@ class Qwen2Model:
         return (ops.gemm_tiles_splitk_count(T, *o, self.dtype),
                 ops.gemm_tiles_splitk_count(T, *down, self.dtype))
 
+    def norm_part_bytes(self, T):
+        """Bytes of the partials _proj_norm leaves for T rows (0: no product splits)."""
+        s = max(self._norm_splits(T))
+        return s * T * self.cfg.hidden_size * 4 if s > 1 else 0
+
     def _proj_norm(self, h, x, weight, gamma, splits):
         """h += x @ weight^T, returns its RMSNorm: the product's k splits into
         the stream's "norm_part" workspace, finished by the norm. None where the

@@ -75,6 +75,13 @@ def test_wide_decode_matches_general_layer(cuda, monkeypatch, B, dtype, graph, h
     r, got, toks = _steps(cuda, B, dtype, graph, head_dim)
     assert r.model_ins_.fused_decode_ok(B) == (B <= model._WIDE_DECODE)
     assert r.model_ins_._norm_splits(5 * B)[1] > 1  # the prefill's down_proj splits
+    if graph and not r.model_ins_.fused_decode_ok(B):
+        # the captured general layer finds the workspace of its split products
+        from lite_lang_amd import ops
+        from lite_lang_amd.models.qwen2.decode_graph import _capture_stream
+        need = r.model_ins_.norm_part_bytes(B)
+        with torch.cuda.stream(_capture_stream(cuda)):
+            assert 0 < need <= ops._WS[ops._ws_key(cuda, "norm_part")].numel()
     monkeypatch.setattr(model, "_WIDE_DECODE", 64)
     monkeypatch.setattr(model.Qwen2Model, "_norm_splits", lambda self, T: (1, 1))
     _, want, _ = _steps(cuda, B, dtype, graph, head_dim, tokens=toks)
